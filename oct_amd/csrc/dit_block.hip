@@ -325,7 +325,7 @@ hipError_t enqueue_dit(const PrometheusDitBlockBf16Request* r, char* ws, const s
                        r->rope_theta, (int)r->rope_axes[0], (int)r->rope_axes[1]);
     PROM_STEP(hipGetLastError());
   }
-  // Each GEMM that runs on the four-stage kernel reads its left operand
+  // Each GEMM that runs on the five-stage kernel reads its left operand
   // K-blocked ([K/32][Tb][32]: whole 128-byte lines per transfer, 4096^3
   // 109 -> 105.5 us), written so by the kernel that produces it; the others
   // read rows.  The values and their order are the same either way.

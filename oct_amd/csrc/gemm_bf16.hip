@@ -13,8 +13,10 @@
 //     one 32-bit LDS store); operand reads are 128-bit;
 //   * exact tails by zero-filled loads and masked stores; the 128-bit global
 //     path needs k % 8 == 0 and n % 8 == 0, other shapes use 16-bit loads.
+// This register-staged kernel is the general one (any alignment and range); the
+// large-tile kernel below and gemm_bf16_tiles.hip serve the rest (bf16_path).
+#include <cmath>
 #include <type_traits>
-
 
 #include "reactor_internal.h"
 
@@ -205,22 +207,17 @@ __global__ __launch_bounds__(256, 2) void gemm_bf16_mfma_kernel(const uint16_t* 
 }
 
 // ---------------------------------------------------------------------------
-// Large-tile kernel: 512 threads = 8 wave64, macro tile 256x256, K tile 64.
-// Waves are 2 (m) x 4 (n); each owns 128x64 = 4x2 MFMA 32x32x16 blocks (128
-// fp32 accumulators per lane).  A stays [m][k] in LDS (operands are 128-bit
-// reads); B stays row-major [k][n] as it arrives from HBM, and each B operand
-// is assembled with two ds_read_b64_tr_b16 transpose reads: within a 16-lane
-// group, lane L points at row (L/4) and column 4*(L%4) of a 4x16 sub-block and
-// receives the 4 k-consecutive values of column L.  No transposing stores.
-// Requires k % 8 == 0, n % 8 == 0 (whole 16-byte chunks are in or out of range).
+// Large-tile kernel: 512 threads = 8 wave64, macro tile 256x256.  Waves are 2 (m)
+// x 4 (n); each owns 128x64 = 4x2 MFMA 32x32x16 blocks (128 fp32 accumulators per
+// lane).  B stays row-major [k][n] as it arrives from HBM, and each B operand is
+// assembled with two ds_read_b64_tr_b16 transpose reads: within a 16-lane group,
+// lane L points at row (L/4) and column 4*(L%4) of a 4x16 sub-block and receives
+// the 4 k-consecutive values of column L.  No transposing stores.
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 
 constexpr int kBM2 = 256;
 constexpr int kBN2 = 256;
-constexpr int kBK2 = 64;
-constexpr int kLdsA2 = kBK2 + 8;   // 144-byte A rows
-constexpr int kLdsB2 = kBN2 + 16;  // 544-byte B rows: 4 consecutive rows land on distinct banks
 
 // Tile (tm, tn) of grouped position pid: groups of kGroupM rows of tiles,
 // column-major inside a group.
@@ -246,342 +243,28 @@ __device__ __forceinline__ void map_tile2(int tiles_m, int tiles_n, int* tm, int
   *tn = in_group / group_m;
 }
 
-template <bool kBuf, int kStoreAt>
-__global__ __launch_bounds__(512, 1) void gemm_bf16_mfma_256_kernel(const uint16_t* __restrict__ A,
-                                                                   const uint16_t* __restrict__ B, float* C, int M,
-                                                                   int N, int K, int tiles_m, int tiles_n, int lda,
-                                                                   int ldb, int ldc, const float* R, int ldr,
-                                                                   uint16_t* Cb) {
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][kBM2][kLdsA2];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][kBK2][kLdsB2];
-
-  int tm, tn;
-  map_tile2(tiles_m, tiles_n, &tm, &tn);
-  const int row0 = tm * kBM2;
-  const int col0 = tn * kBN2;
-  const int tid = (int)threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wm = wave >> 2;  // 0..1
-  const int wn = wave & 3;   // 0..3
-
-  u32x4 ra[4], rb[4];
-  // Branch-free path (kBuf): buffer loads return zero past the end of A or B, which
-  // covers rows >= M and k >= K (K is a multiple of the K tile there); columns >= N
-  // read the next row of B but only feed output columns that are never stored.
-  const __amdgpu_buffer_rsrc_t rsa =
-      __builtin_amdgcn_make_buffer_rsrc((void*)A, (short)0, kBuf ? (int)((size_t)M * lda * 2) : 0, 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)B, (short)0, kBuf ? (int)((size_t)K * ldb * 2) : 0, 0x00020000);
-  auto load_tile = [&](int k0) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = tid + 512 * u;  // A: 256 rows x 8 chunks
-      const int r = c >> 3;
-      const int kc = (c & 7) * 8;
-      const int gr = row0 + r, gk = k0 + kc;
-      if constexpr (kBuf) {
-        ra[u] = __builtin_amdgcn_raw_buffer_load_b128(rsa, (uint32_t)((gr * lda + gk) * 2), 0, 0);
-      } else {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (gr < M && gk < K) v = *reinterpret_cast<const u32x4*>(A + (size_t)gr * lda + gk);
-        ra[u] = v;
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = tid + 512 * u;  // B: 64 k rows x 32 chunks
-      const int kr = c >> 5;
-      const int nc = (c & 31) * 8;
-      const int gk = k0 + kr, gn = col0 + nc;
-      if constexpr (kBuf) {
-        rb[u] = __builtin_amdgcn_raw_buffer_load_b128(rsb, (uint32_t)((gk * ldb + gn) * 2), 0, 0);
-      } else {
-        u32x4 v = {0u, 0u, 0u, 0u};
-        if (gk < K && gn < N) v = *reinterpret_cast<const u32x4*>(B + (size_t)gk * ldb + gn);
-        rb[u] = v;
-      }
-    }
-  };
-  auto store_tile = [&](int buf) {
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = tid + 512 * u;
-      *reinterpret_cast<u32x4*>(&As[buf][c >> 3][(c & 7) * 8]) = ra[u];
-    }
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int c = tid + 512 * u;
-      *reinterpret_cast<u32x4*>(&Bs[buf][c >> 5][(c & 31) * 8]) = rb[u];
-    }
-  };
-
-  floatx16 acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i][0] = floatx16{};
-    acc[i][1] = floatx16{};
-  }
-
-  const int k_tiles = (K + kBK2 - 1) / kBK2;
-  load_tile(0);
-  store_tile(0);
-  __syncthreads();
-
-  const int lrow = lane & 31;
-  const int lk = (lane >> 5) * 8;
-  // transpose-read coordinates inside a 16(k) x 32(n) operand block
-  const int tr_row = 8 * (lane >> 5) + ((lane & 15) >> 2);
-  const int tr_col = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    const int cur = kt & 1;
-    const bool more = kt + 1 < k_tiles;
-    if (more) load_tile((kt + 1) * kBK2);
-#pragma unroll
-    for (int s = 0; s < kBK2 / 16; ++s) {
-      bf16x8 af[4], bfr[2];
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
-        af[mi] = *reinterpret_cast<const bf16x8*>(&As[cur][wm * 128 + mi * 32 + lrow][16 * s + lk]);
-#pragma unroll
-      for (int ni = 0; ni < 2; ++ni) {
-        const int col = wn * 64 + ni * 32 + tr_col;
-        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s16x4*)(&Bs[cur][16 * s + tr_row][col]));
-        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-            (lds_s16x4*)(&Bs[cur][16 * s + tr_row + 4][col]));
-        const short w8[8] = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        bfr[ni] = __builtin_bit_cast(bf16x8, w8);
-      }
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[mi], bfr[ni], acc[mi][ni], 0, 0, 0);
-      }
-      // The other buffer was last read before the previous barrier, so the next
-      // tile may be written into it at any point of this iteration.
-      if (s == kStoreAt && more) store_tile(cur ^ 1);
-    }
-    __syncthreads();
-  }
-
-  const int lgrp = (lane >> 5) * 4;
-#pragma unroll
-  for (int mi = 0; mi < 4; ++mi) {
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      const int col = col0 + wn * 64 + ni * 32 + lrow;
-      if (col >= N) continue;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int row = row0 + wm * 128 + mi * 32 + 8 * (r >> 2) + lgrp + (r & 3);
-        if (row < M) {
-          float v = acc[mi][ni][r];
-          if (R != nullptr) v += R[(size_t)row * ldr + col];
-          if (Cb != nullptr)
-            Cb[(size_t)row * ldc + col] = f32_to_bf16_rne(v);
-          else
-            C[(size_t)row * ldc + col] = v;
-        }
-      }
-    }
-  }
-}
-
-// Direct-to-LDS variant of the 8-wave large tile.  Tiles travel HBM -> LDS
-// with buffer_load_dwordx4 ... lds (no staging registers, no ds_write), so
-// tile kt+1 streams into the other stage during all of tile kt's MFMAs.  Each
-// wave instruction fills 1 KiB of LDS, lane i at +16*i, which fixes an
-// unpadded layout; the global address each lane fetches applies an XOR
-// swizzle on 16-byte chunks so that the MFMA operand reads are bank-conflict
-// free: A (256 x 64, 128-byte rows) chunk c of row R sits at c ^ ((R&7) ^ ((R>>3)&1)),
-// B (64 x 256, 512-byte rows) chunk c of row k at c ^ {0,4,10,14}[k&3].
-// The two stages are separate LDS arrays and the K loop is unrolled by two so
-// that reads of one stage are visibly independent of the DMA into the other.
-__device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 3) & 1); }
+// Tiles travel HBM -> LDS with buffer_load_dwordx4 ... lds (no staging registers, no
+// ds_write).  Each wave instruction fills 1 KiB of LDS, lane i at +16*i, which
+// fixes an unpadded layout; the global address each lane fetches applies an XOR
+// swizzle on 16-byte chunks so that the operand reads are bank-conflict free: chunk
+// c of A row R (64 bytes) sits at c ^ ((R >> 2) & 3), chunk c of B row k (512 bytes)
+// at c ^ {0,4,10,14}[k & 3].
 __device__ __forceinline__ int swz_b(int k) { return (0xEA40 >> (4 * (k & 3))) & 15; }  // {0,4,10,14}
 
+// K tile 32, five 32 KB LDS stages (the whole 160 KB), so each tile's transfers are
+// issued four tiles ahead of its MFMAs (one 32-k step of the whole tile takes
+// ~1000-1800 cycles per SIMD, the HBM and Infinity Cache latency is longer; five
+// stages measured 1-3 % faster than four at 4224 x 11520 x 3840 and 8192^3).
+// Waits count this wave's outstanding transfers (4 per tile) and a bare
+// s_barrier publishes a tile: transfers of the next tiles stay in flight
+// across it.  It runs where the shape fills the chip with 256x256 tiles; other
+// shapes take the tiles of gemm_bf16_tiles.hip (bf16_path).
 //
 // kSwiGLU: B is [K, 2F] = [W1 | W3] and the output is h = silu(x W1) * (x W3)
 // in bf16 [M, F].  A tile then covers 128 output columns: in each wave's 64
 // B columns the first 32 are gate (W1) columns and the last 32 the matching
 // up (W3) columns, so accumulator blocks ni = 0 and 1 hold g and u of the same
 // outputs and the product is formed in registers (N is F here).
-template <bool kSwiGLU>
-__global__ __launch_bounds__(512, 1) void gemm_bf16_mfma_dl_kernel(const uint16_t* __restrict__ A,
-                                                                  const uint16_t* __restrict__ B, float* C, int M,
-                                                                  int N, int K, int tiles_m, int tiles_n, int lda,
-                                                                  int ldb, int ldc, const float* R, int ldr,
-                                                                  uint16_t* Cb) {
-  __shared__ __attribute__((aligned(1024))) uint16_t S0[2 * kBM2 * kBK2];
-  __shared__ __attribute__((aligned(1024))) uint16_t S1[2 * kBM2 * kBK2];
-
-  int tm, tn;
-  map_tile2(tiles_m, tiles_n, &tm, &tn);
-  const int row0 = tm * kBM2;
-  const int col0 = kSwiGLU ? tn * (kBN2 / 2) : tn * kBN2;
-  const int tid = (int)threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave >> 2;
-  const int wn = wave & 3;
-
-  const __amdgpu_buffer_rsrc_t rsa =
-      __builtin_amdgcn_make_buffer_rsrc((void*)A, (short)0, (int)((size_t)M * lda * 2), 0x00020000);
-  const __amdgpu_buffer_rsrc_t rsb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)B, (short)0, (int)((size_t)K * ldb * 2), 0x00020000);
-
-  // Per-lane source offsets (bytes) of this wave's 4 A and 4 B instructions at
-  // k0 = 0; the k offset of a tile travels in the scalar soffset.
-  uint32_t a_off[4], b_off[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int q = wave * 4 + i;
-    const int r = 8 * q + (lane >> 3);
-    const int c = (lane & 7) ^ swz_a(r);
-    a_off[i] = (uint32_t)(((row0 + r) * lda + 8 * c) * 2);
-    const int kr = 2 * q + (lane >> 5);
-    const int cb = (lane & 31) ^ swz_b(kr);
-    int gcol = col0 + 8 * cb;
-    if constexpr (kSwiGLU) {
-      const int e = 8 * cb;  // tile column: wave block e / 64, gate half if e % 64 < 32
-      gcol = col0 + (e >> 6) * 32 + (e & 31) + ((e & 32) ? N : 0);
-    }
-    b_off[i] = (uint32_t)((kr * ldb + gcol) * 2);
-  }
-  typedef __attribute__((address_space(3))) void lds_void;
-  auto issue = [&](uint16_t* stage, int k0) {
-    const int sa = __builtin_amdgcn_readfirstlane(k0 * 2);
-    const int sb = __builtin_amdgcn_readfirstlane(k0 * ldb * 2);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int q = wave * 4 + i;
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsa, (lds_void*)((char*)stage + q * 1024), 16, a_off[i], sa, 0, 0);
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_void*)((char*)stage + 32768 + q * 1024), 16, b_off[i], sb,
-                                               0, 0);
-    }
-  };
-
-  // Operand addresses.  A row R = wm*128 + mi*32 + lrow has swizzle swz_a(lrow)
-  // for every mi, and chunk 2s + hk = 2s ^ hk, so the byte address of step s is
-  // a_base ^ (32 s) plus the immediate mi*4096.  B rows 16s + tr_row (+4) share
-  // swizzle swz_b(tr_row); chunk (wn*8 + 4ni + x) ^ sw = ((wn*8 + x) ^ sw) ^ 4ni,
-  // so its address is b_base ^ (64 ni) plus the immediates 8192 s (+2048).
-  const int lrow = lane & 31;
-  const int hk = lane >> 5;
-  const int tr_row = 8 * (lane >> 5) + ((lane & 15) >> 2);
-  const int tr_e = 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
-  const uint32_t a_base = (uint32_t)((wm * 128 + lrow) * 128 + ((hk ^ swz_a(lrow)) << 4));
-  const uint32_t b_base =
-      (uint32_t)(32768 + tr_row * 512 + (((wn * 8 + (tr_e >> 3)) ^ swz_b(tr_row)) << 4) + (tr_e & 7) * 2);
-  struct Frags {
-    bf16x8 a[4], b[2];
-  };
-  auto read_frags = [&](const uint16_t* stage, int s) {
-    Frags f;
-    const char* st = (const char*)stage;
-    const uint32_t as = a_base ^ (uint32_t)(32 * s);
-#pragma unroll
-    for (int mi = 0; mi < 4; ++mi) f.a[mi] = *reinterpret_cast<const bf16x8*>(st + as + mi * 4096);
-#pragma unroll
-    for (int ni = 0; ni < 2; ++ni) {
-      const uint32_t bs = (b_base ^ (uint32_t)(64 * ni)) + 8192 * s;
-      const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(st + bs));
-      const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(st + bs + 2048));
-      f.b[ni] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-    }
-    return f;
-  };
-
-  floatx16 acc[4][2];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i][0] = floatx16{};
-    acc[i][1] = floatx16{};
-  }
-  auto compute = [&](const uint16_t* stage) {
-#pragma unroll
-    for (int s = 0; s < kBK2 / 16; ++s) {
-      const Frags fc = read_frags(stage, s);
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-          acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fc.a[mi], fc.b[ni], acc[mi][ni], 0, 0, 0);
-    }
-  };
-
-  const int k_tiles = K / kBK2;
-  issue(S0, 0);
-  __builtin_amdgcn_s_waitcnt(0);
-  __syncthreads();
-  for (int kt = 0; kt < k_tiles; ++kt) {
-    // stage kt&1 holds tile kt; the other stage was last read before the previous barrier
-    uint16_t* cur = (kt & 1) ? S1 : S0;
-    uint16_t* nxt = (kt & 1) ? S0 : S1;
-    if (kt + 1 < k_tiles) issue(nxt, (kt + 1) * kBK2);
-    compute(cur);
-    __builtin_amdgcn_s_waitcnt(0);
-    __syncthreads();
-  }
-
-  const int lgrp = (lane >> 5) * 4;
-  if constexpr (kSwiGLU) {
-    const int col = col0 + wn * 32 + lrow;
-    if (col < N) {
-#pragma unroll
-      for (int mi = 0; mi < 4; ++mi) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int row = row0 + wm * 128 + mi * 32 + 8 * (r >> 2) + lgrp + (r & 3);
-          if (row < M) {
-            const float g = acc[mi][0][r], u = acc[mi][1][r];
-            Cb[(size_t)row * ldc + col] = f32_to_bf16_rne(silu_mul(g, u));
-          }
-        }
-      }
-    }
-    return;
-  }
-  auto store_block = [&](const floatx16& v16, int mi, int ni) {
-    const int col = col0 + wn * 64 + ni * 32 + lrow;
-    if (col >= N) return;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int row = row0 + wm * 128 + mi * 32 + 8 * (r >> 2) + lgrp + (r & 3);
-      if (row < M) {
-        float v = v16[r];
-        if (R != nullptr) v += R[(size_t)row * ldr + col];
-        if (Cb != nullptr)
-          Cb[(size_t)row * ldc + col] = f32_to_bf16_rne(v);
-        else
-          C[(size_t)row * ldc + col] = v;
-      }
-    }
-  };
-  store_block(acc[0][0], 0, 0);
-  store_block(acc[0][1], 0, 1);
-  store_block(acc[1][0], 1, 0);
-  store_block(acc[1][1], 1, 1);
-  store_block(acc[2][0], 2, 0);
-  store_block(acc[2][1], 2, 1);
-  store_block(acc[3][0], 3, 0);
-  store_block(acc[3][1], 3, 1);
-}
-
-// Multi-stage variant of the direct-to-LDS kernel: K tile 32, five 32 KB LDS
-// stages (the whole 160 KB), so each tile's transfers are issued four tiles
-// ahead of its MFMAs (one 32-k step of the whole tile takes ~1000-1800 cycles
-// per SIMD, the HBM and Infinity Cache latency is longer; five stages
-// measured 1-3 % faster than four on the C5 shapes and 8192^3).  A rows are 64 bytes here: chunk c of row
-// R sits at c ^ ((R >> 2) & 3); B keeps the 512-byte rows and swizzle above.
-// Waits count this wave's outstanding transfers (4 per tile) and a bare
-// s_barrier publishes a tile: transfers of the next tiles stay in flight
-// across it.  Faster than the two-stage kernel on long K and on grids of more
-// than one workgroup per CU (C5's QKV, W1|W3 and W2 products, 8192^3: 6-16 %),
-// slower on single-round grids with K <= 4096 (4096^3: -9 %).
 constexpr int kBK4 = 32;
 constexpr int kStage4 = kBM2 * kBK4 * 2 + kBK4 * kBN2 * 2;  // 16 KB A + 16 KB B
 
@@ -626,7 +309,9 @@ __device__ __forceinline__ void gemm_bf16_dl4_body(const uint16_t* __restrict__ 
       const int e = 8 * cb;
       gcol = col0 + (e >> 6) * 32 + (e & 31) + ((e & 32) ? N : 0);
     }
-    b_off[i] = (uint32_t)((kr * ldb + gcol) * 2);
+    // Columns past N feed only outputs that are never stored; out of the descriptor's
+    // range they are not read at all (the last row's would lie past the end of B).
+    b_off[i] = !kSwiGLU && gcol >= N ? 0x80000000u : (uint32_t)((kr * ldb + gcol) * 2);
   }
   // The transfers are written as inline assembly (M0 = LDS destination of
   // the wave's 1 KB, 16 bytes per lane; buffer descriptors built here, raw,
@@ -907,34 +592,58 @@ __global__ __launch_bounds__(256) void swiglu_splitk_kernel(const float2* __rest
 
 inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
-// The four-stage kernel wins once a CU runs more than one tile in turn or the
-// K loop is long (measured on MI355X; see its comment).
-// The multi-stage kernel from 240 tiles (C5's 255-tile output projection:
-// 115.3 -> 111.7 us) or K >= 8192.
-inline bool use_four_stage(int tiles, uint32_t k) { return tiles >= 240 || k >= 8192; }
-
 }  // namespace
 
 namespace {
 
-enum class Bf16Path { kFourStage, kTwoStage, kStaged256, kSmall };
+enum class Bf16Path { kFiveStage, kTiles, kPadded, kSmall };
 
-// The kernel launch_gemm_bf16_ex runs for a shape and its operands' layout.
+// The kernel launch_gemm_bf16_ex runs for a shape and its operands' layout: the
+// least estimate of the 256x256 five-stage kernel (whole K tiles of 32 only) and
+// the tiles of gemm_bf16_tiles.hip.  Operands without 16-byte rows are first copied
+// to zero-padded buffers, unless the product is so small that the launches cost
+// more than the register-staged kernel's 16-bit loads (about 5.5 us per K tile of
+// 64 there: 1023x2049x777 82 us, 33x3001x5003 324 us).
 Bf16Path bf16_path(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n, uint32_t k,
-                   bool* vec_out) {
-  const bool vec = (k % 8 == 0) && (n % 8 == 0) && (lda % 8 == 0) && (ldb % 8 == 0) && aligned16(a) && aligned16(b);
-  if (vec_out) *vec_out = vec;
-  const int tiles = (int)((m + kBM2 - 1) / kBM2) * (int)((n + kBN2 - 1) / kBN2);
-  if (!vec || tiles < 128) return Bf16Path::kSmall;
-  const bool range = (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * ldb * 2 < (1ull << 31);
-  if (range && k % kBK4 == 0 && use_four_stage(tiles, k)) return Bf16Path::kFourStage;
-  if (range && k % kBK2 == 0) return Bf16Path::kTwoStage;
-  return Bf16Path::kStaged256;
+                   Bf16TilePlan* plan) {
+  *plan = plan_bf16_tiles(m, n, k, false);
+  if (bf16_tiles_take(a, lda, b, ldb, k)) {
+    const bool range = (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * ldb * 2 < (1ull << 31);
+    return range && k % kBK4 == 0 && bf16_five_stage_us(m, n, k, 0) < plan->us ? Bf16Path::kFiveStage
+                                                                                  : Bf16Path::kTiles;
+  }
+  if (k >= (1u << 22) - 8 || n >= (1u << 23) - 8) return Bf16Path::kSmall;
+  const double tiles128 = (double)((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
+  const double small_us = 4.0 + std::ceil(tiles128 / 512.0) * std::ceil(k / 64.0) * 5.5;
+  const double padded_us = plan->us + 7.0 + 4.0 * ((double)m * k + (double)k * n) / 3.0e6;
+  return small_us < padded_us ? Bf16Path::kSmall : Bf16Path::kPadded;
 }
 
-bool swiglu_fused_ok(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f, uint32_t k) {
+bool swiglu_five_stage_ok(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f, uint32_t k) {
   return f % 128 == 0 && k % kBK4 == 0 && lda % 8 == 0 && aligned16(a) && aligned16(w13) &&
          (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * 2 * f * 2 < (1ull << 31);
+}
+
+bool swiglu_tiles_ok(const uint16_t* a, int lda, const uint16_t* w13, uint32_t f, uint32_t k) {
+  return f % 8 == 0 && bf16_tiles_take(a, lda, w13, (int)(2 * f), k);
+}
+
+// K slices of the tiles of a final wave that would run at most half full (0 or 1: none).
+int swiglu_tail_splits(uint32_t m, uint32_t f, uint32_t k) {
+  const int total = (int)((m + kBM2 - 1) / kBM2) * (int)(f / 128);
+  const int cus = ctx().props.multiProcessorCount > 0 ? ctx().props.multiProcessorCount : 256;
+  const int rem = total % cus;
+  const int splits = rem > 0 ? std::min(cus / rem, 4) : 0;
+  return total > cus && splits >= 2 && (int)(k / kBK4) >= 4 * splits ? splits : 0;
+}
+
+// True when the SwiGLU GEMM runs on the five-stage kernel, as bf16_path decides.  Where
+// its final wave is split along K the estimate, which adds the waves up, is too
+// high (dispatch overlaps them), so there the tiles have to be 30 % better.
+bool swiglu_five_stage(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f, uint32_t k) {
+  if (!swiglu_five_stage_ok(a, lda, w13, m, f, k)) return false;
+  const int splits = swiglu_tail_splits(m, f, k);
+  return bf16_five_stage_us(m, 2 * f, k, splits) < plan_bf16_tiles(m, 2 * f, k, true).us * (splits >= 2 ? 1.3 : 1.0);
 }
 
 // K-blocked A ([k/32][a_slice][32], a_slice >= m rounded up to 256 rows) keeps
@@ -947,47 +656,64 @@ bool blocked_range(int a_slice, uint32_t m, uint32_t k) {
 
 bool gemm_bf16_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n,
                                uint32_t k) {
-  return bf16_path(a, lda, b, ldb, m, n, k, nullptr) == Bf16Path::kFourStage;
+  Bf16TilePlan plan;
+  return bf16_path(a, lda, b, ldb, m, n, k, &plan) == Bf16Path::kFiveStage;
 }
 
 bool gemm_bf16_swiglu_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f,
                                       uint32_t k) {
-  const int tiles = (int)((m + kBM2 - 1) / kBM2) * (int)(f / 128);
-  return swiglu_fused_ok(a, lda, w13, m, f, k) && use_four_stage(tiles, k);
+  return swiglu_five_stage(a, lda, w13, m, f, k);
 }
 
 hipError_t launch_gemm_bf16_ex(const uint16_t* a, int lda, const uint16_t* b, int ldb, float* c, uint16_t* cb,
                                int ldc, uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr,
                                hipStream_t stream, int* path_detail, int a_slice) {
-  bool vec = false;
-  const Bf16Path path = bf16_path(a, lda, b, ldb, m, n, k, &vec);
-  if (a_slice > 0 && (path != Bf16Path::kFourStage || !blocked_range(a_slice, m, k))) return hipErrorNotSupported;
-  if (path != Bf16Path::kSmall) {
+  Bf16TilePlan plan;
+  Bf16Path path = bf16_path(a, lda, b, ldb, m, n, k, &plan);
+  if (a_slice > 0 && (path != Bf16Path::kFiveStage || !blocked_range(a_slice, m, k))) return hipErrorNotSupported;
+  if (path_detail) *path_detail = PROM_DETAIL_PATH_HIP_MFMA_BF16;
+  if (path == Bf16Path::kFiveStage) {
     const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
     const int tiles_n2 = (int)((n + kBN2 - 1) / kBN2);
-    const dim3 grid2((unsigned)(tiles_m2 * tiles_n2));
-    if (path == Bf16Path::kFourStage)
-      hipLaunchKernelGGL(gemm_bf16_dl4_kernel, grid2, dim3(512), 0, stream, a, b, c, (int)m, (int)n, (int)k, tiles_m2,
-                         tiles_n2, lda, ldb, ldc, residual, ldr, cb, a_slice);
-    else if (path == Bf16Path::kTwoStage)
-      hipLaunchKernelGGL(gemm_bf16_mfma_dl_kernel<false>, grid2, dim3(512), 0, stream, a, b, c, (int)m, (int)n, (int)k,
-                         tiles_m2, tiles_n2, lda, ldb, ldc, residual, ldr, cb);
-    else
-      hipLaunchKernelGGL((gemm_bf16_mfma_256_kernel<false, 1>), grid2, dim3(512), 0, stream, a, b, c, (int)m, (int)n,
-                         (int)k, tiles_m2, tiles_n2, lda, ldb, ldc, residual, ldr, cb);
-    if (path_detail) *path_detail = PROM_DETAIL_PATH_HIP_MFMA_BF16;
+    hipLaunchKernelGGL(gemm_bf16_dl4_kernel, dim3((unsigned)(tiles_m2 * tiles_n2)), dim3(512), 0, stream, a, b, c,
+                       (int)m, (int)n, (int)k, tiles_m2, tiles_n2, lda, ldb, ldc, residual, ldr, cb, a_slice);
     return hipGetLastError();
   }
+  if (path == Bf16Path::kPadded) {
+    const bool copy_a = k % 8 != 0 || lda % 8 != 0 || !aligned16(a);
+    const bool copy_b = ldb % 8 != 0 || !aligned16(b);
+    const int k8 = (int)((k + 7u) & ~7u), n8 = (int)((n + 7u) & ~7u);
+    uint16_t* pa = copy_a ? static_cast<uint16_t*>(staging(8, (size_t)m * k8 * 2)) : nullptr;
+    uint16_t* pb = copy_b ? static_cast<uint16_t*>(staging(9, (size_t)k * n8 * 2)) : nullptr;
+    if ((copy_a && pa == nullptr) || (copy_b && pb == nullptr)) {
+      path = Bf16Path::kSmall;  // no room for the copies
+    } else {
+      hipError_t e = hipSuccess;
+      if (copy_a) e = launch_bf16_pad_rows(a, pa, m, k, lda, k8, stream);
+      if (e == hipSuccess && copy_b) e = launch_bf16_pad_rows(b, pb, k, n, ldb, n8, stream);
+      if (e != hipSuccess) return e;
+      if (copy_a) {
+        a = pa;
+        lda = k8;
+      }
+      if (copy_b) {
+        b = pb;
+        ldb = n8;
+      }
+    }
+  }
+  if (path != Bf16Path::kSmall)
+    return launch_bf16_tiles(plan, false, a, lda, b, ldb, c, cb, ldc, m, n, k, residual, ldr, stream);
   const int tiles_m = (int)((m + kBM - 1) / kBM);
   const int tiles_n = (int)((n + kBN - 1) / kBN);
   const dim3 grid((unsigned)(tiles_m * tiles_n));
+  const bool vec = k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned16(a) && aligned16(b);
   if (vec)
     hipLaunchKernelGGL(gemm_bf16_mfma_kernel<true>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
                        tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
   else
     hipLaunchKernelGGL(gemm_bf16_mfma_kernel<false>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
                        tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
-  if (path_detail) *path_detail = PROM_DETAIL_PATH_HIP_MFMA_BF16;
   return hipGetLastError();
 }
 
@@ -995,48 +721,44 @@ hipError_t launch_gemm_bf16_swiglu(const uint16_t* a, int lda, const uint16_t* w
                                    uint32_t f, uint32_t k, hipStream_t stream, void* part_ws, size_t part_bytes,
                                    uint32_t* launches, int a_slice, int h_slice) {
   if (launches) *launches = 1;
-  // Fused path conditions: whole 128-column output tiles, K a multiple of the K
-  // tile, 16-byte aligned rows, byte offsets below 2^31; otherwise the caller
-  // runs the GEMM and the elementwise SwiGLU separately.
-  if (!swiglu_fused_ok(a, lda, w13, m, f, k)) return hipErrorNotSupported;
+  // Fused path conditions: 16-byte aligned rows and byte offsets below 2^31;
+  // otherwise the caller runs the GEMM and the elementwise SwiGLU separately.
+  if (!swiglu_five_stage(a, lda, w13, m, f, k)) {
+    if (a_slice > 0 || h_slice > 0) return hipErrorInvalidValue;
+    if (!swiglu_tiles_ok(a, lda, w13, f, k)) return hipErrorNotSupported;
+    return launch_bf16_tiles(plan_bf16_tiles(m, 2 * f, k, true), true, a, lda, w13, (int)(2 * f), nullptr, h, ldh, m,
+                             f, k, nullptr, 0, stream);
+  }
   const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
   const int tiles_n2 = (int)(f / 128);
   const dim3 grid((unsigned)(tiles_m2 * tiles_n2));
-  const bool four = use_four_stage(tiles_m2 * tiles_n2, k);
-  // K-blocked A or H only on the four-stage kernel.
-  if ((a_slice > 0 && (!four || !blocked_range(a_slice, m, k))) ||
-      (h_slice > 0 && (!four || h_slice < tiles_m2 * kBM2 || (size_t)f * h_slice * 2 >= (1ull << 31))))
+  // K-blocked A or H.
+  if ((a_slice > 0 && !blocked_range(a_slice, m, k)) ||
+      (h_slice > 0 && (h_slice < tiles_m2 * kBM2 || (size_t)f * h_slice * 2 >= (1ull << 31))))
     return hipErrorInvalidValue;
-  if (four) {
-    // One workgroup per CU: the tiles of a final wave that would run at most
-    // half full are split along K into as many slices as fill it (at most 4,
-    // each of 4 K tiles or more), their partial sums going to part_ws.
-    const int total = tiles_m2 * tiles_n2;
-    const int cus = ctx().props.multiProcessorCount > 0 ? ctx().props.multiProcessorCount : 256;
-    const int rem = total % cus;
-    const int splits = rem > 0 ? std::min(cus / rem, 4) : 0;
-    const int k_tiles = (int)(k / kBK4);
-    const size_t need = (size_t)rem * splits * kBM2 * 128 * sizeof(float2);
-    if (total > cus && splits >= 2 && k_tiles >= 4 * splits && part_ws != nullptr && need <= part_bytes) {
-      const int n_main = total - rem;
-      hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, dim3((unsigned)(n_main + rem * splits)), dim3(512), 0, stream, a,
-                         w13, (int)m, (int)f, (int)k, tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, n_main, splits,
-                         reinterpret_cast<float2*>(part_ws), a_slice, h_slice);
-      const hipError_t e = hipGetLastError();
-      if (e != hipSuccess) return e;
-      hipLaunchKernelGGL(swiglu_splitk_kernel, dim3(kBM2 * 128 / 256, (unsigned)rem), dim3(256), 0, stream,
-                         reinterpret_cast<const float2*>(part_ws), h, ldh, (int)m, tiles_m2, tiles_n2, n_main, splits,
-                         h_slice);
-      if (launches) *launches = 2;
-    } else {
-      hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, grid, dim3(512), 0, stream, a, w13, (int)m, (int)f, (int)k,
-                         tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, total, 1, nullptr, a_slice, h_slice);
-    }
-  } else if (k % kBK2 == 0)
-    hipLaunchKernelGGL(gemm_bf16_mfma_dl_kernel<true>, grid, dim3(512), 0, stream, a, w13, nullptr, (int)m, (int)f,
-                       (int)k, tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, nullptr, 0, h);
-  else
-    return hipErrorNotSupported;
+  // One workgroup per CU: the tiles of a final wave that would run at most
+  // half full are split along K into as many slices as fill it (at most 4,
+  // each of 4 K tiles or more), their partial sums going to part_ws.
+  const int total = tiles_m2 * tiles_n2;
+  const int cus = ctx().props.multiProcessorCount > 0 ? ctx().props.multiProcessorCount : 256;
+  const int rem = total % cus;
+  const int splits = swiglu_tail_splits(m, f, k);
+  const size_t need = (size_t)rem * splits * kBM2 * 128 * sizeof(float2);
+  if (splits >= 2 && part_ws != nullptr && need <= part_bytes) {
+    const int n_main = total - rem;
+    hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, dim3((unsigned)(n_main + rem * splits)), dim3(512), 0, stream, a,
+                       w13, (int)m, (int)f, (int)k, tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, n_main, splits,
+                       reinterpret_cast<float2*>(part_ws), a_slice, h_slice);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(swiglu_splitk_kernel, dim3(kBM2 * 128 / 256, (unsigned)rem), dim3(256), 0, stream,
+                       reinterpret_cast<const float2*>(part_ws), h, ldh, (int)m, tiles_m2, tiles_n2, n_main, splits,
+                       h_slice);
+    if (launches) *launches = 2;
+  } else {
+    hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, grid, dim3(512), 0, stream, a, w13, (int)m, (int)f, (int)k,
+                       tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, total, 1, nullptr, a_slice, h_slice);
+  }
   return hipGetLastError();
 }
 

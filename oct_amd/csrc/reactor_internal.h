@@ -62,7 +62,7 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 constexpr uint64_t kRuntimeMagic = 0x4F43544D49333535ull;  // "OCTMI355"
 constexpr uint32_t kEventSlots = 64;
 // Staging slots: 0-3 operand staging, 4 block workspace, 5 block host staging,
-// 6 split-K partials, 7 FFT twiddle table, 8-9 padded SGEMM operand copies.
+// 6 split-K partials, 7 FFT twiddle table, 8-9 padded GEMM operand copies.
 constexpr uint32_t kStagingSlots = 10;
 
 struct AsyncState;  // async task table, submission slots and batch arenas (sgemm_async.hip)
@@ -196,17 +196,17 @@ hipError_t launch_sgemm_f32_batched(const float* a, int lda, long long sa, const
 // K-blocked A: a_slice > 0 says A is stored as [k/32][a_slice][32] (the 32
 // consecutive k of one row are 64 contiguous bytes, rows of a slice adjacent,
 // a_slice >= m rounded up to 256), so every HBM -> LDS transfer of A moves
-// whole 128-byte lines; only the four-stage kernel reads it, and
+// whole 128-byte lines; only the five-stage kernel reads it, and
 // gemm_bf16_takes_blocked_a says whether a shape runs there (with a_slice == 0
 // A is row-major with row stride lda).  hipErrorNotSupported otherwise.
 hipError_t launch_gemm_bf16_ex(const uint16_t* a, int lda, const uint16_t* b, int ldb, float* c, uint16_t* cb,
                                int ldc, uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr,
                                hipStream_t stream, int* path_detail, int a_slice = 0);
-// True when launch_gemm_bf16_ex runs this shape on the four-stage kernel (a:
+// True when launch_gemm_bf16_ex runs this shape on the five-stage kernel (a:
 // 16-byte aligned, lda its row-major stride).
 bool gemm_bf16_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n,
                                uint32_t k);
-// The same for the fused SwiGLU GEMM, whose four-stage kernel also writes H
+// The same for the fused SwiGLU GEMM, whose five-stage kernel also writes H
 // K-blocked ([f/32][h_slice][32]) for a following GEMM when h_slice > 0.
 bool gemm_bf16_swiglu_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f,
                                       uint32_t k);
@@ -223,6 +223,25 @@ hipError_t launch_gemm_bf16(const uint16_t* a, const uint16_t* b, float* c, uint
 hipError_t launch_gemm_bf16_swiglu(const uint16_t* a, int lda, const uint16_t* w13, uint16_t* h, int ldh, uint32_t m,
                                    uint32_t f, uint32_t k, hipStream_t stream, void* part_ws, size_t part_bytes,
                                    uint32_t* launches = nullptr, int a_slice = 0, int h_slice = 0);
+// The multi-tile bf16 GEMM (gemm_bf16_tiles.hip).  plan_bf16_tiles picks the
+// macro tile and the K slices with the least estimated time for C[m, n] (swiglu:
+// n = 2f weight columns); launch_bf16_tiles runs a plan (swiglu: n = f, cb the
+// bf16 output) on operands bf16_tiles_take accepts (16-byte aligned rows, k % 8 ==
+// 0); k need not be a multiple of 8 when A's rows are zero-padded to one
+// (launch_bf16_pad_rows).  bf16_five_stage_us estimates the 256x256 kernel of
+// gemm_bf16.hip by the same model, tail_splits >= 2: its final wave split along K.
+struct Bf16TilePlan {
+  int tile, splits;
+  double us;
+};
+Bf16TilePlan plan_bf16_tiles(uint32_t m, uint32_t n, uint32_t k, bool swiglu);
+double bf16_five_stage_us(uint32_t m, uint32_t n, uint32_t k, int tail_splits);
+bool bf16_tiles_take(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t k);
+hipError_t launch_bf16_tiles(Bf16TilePlan plan, bool swiglu, const uint16_t* a, int lda, const uint16_t* b, int ldb,
+                             float* c, uint16_t* cb, int ldc, uint32_t m, uint32_t n, uint32_t k,
+                             const float* residual, int ldr, hipStream_t stream);
+hipError_t launch_bf16_pad_rows(const uint16_t* src, uint16_t* dst, uint32_t rows, uint32_t cols, int ld_s, int ld_d,
+                                hipStream_t stream);
 // bf16 flash attention, head dim 128, full (non-causal): Q/K/V/O [T, ld*] with
 // head h at column 128 h.  variant 0: K/V tiles moved HBM -> LDS by DMA (64 KiB
 // of dynamic LDS); 1: tiles staged through registers.  hipErrorInvalidValue for
