@@ -441,25 +441,28 @@ constexpr int kTileK = 64;
 // does not fill the chip the step falls towards `idle` of it.  The constants are
 // a least-squares fit (log time) to 1859 (tile, K slices) runs at 58 shapes on
 // MI355X, m 32..4224, n 256..11520, k 256..10240: rms 4.4 %, and the plan with
-// the least estimate is within 2 % of the fastest measured on average (the worst
-// of the 58 loses 20 %: 32x11520x10240, bound by reading B).
+// the least estimate is within 2 % of the fastest measured on average, 15 % at worst.
+// A large B (past what the caches hold) is read at the rate its bytes in flight
+// allow: `flight` KiB per workgroup over ~1.5 us of latency, 5 TB/s at most
+// (32x11520x10240, one K slice of 64x64 tiles 72 us, four of 64x256 46 us).
 struct TileCost {
   int occ;
-  double step[2], fill, idle;
+  double step[2], fill, idle, flight;
 };
 constexpr TileCost kCost[kNumTiles + 1] = {
-    {2, {0.203, 0.452}, 2.36, 0.86},  // 32x128
-    {2, {0.190, 0.375}, 2.49, 0.77},  // 64x64
-    {2, {0.325, 0.648}, 2.84, 0.58},  // 64x128
-    {1, {0.639, 0.639}, 3.49, 0.41},  // 64x256
-    {1, {0.585, 0.585}, 3.49, 0.46},  // 128x128
-    {1, {0.740, 0.740}, 5.24, 0.36},  // 192x128
-    {1, {0.945, 0.945}, 5.67, 0.42},  // 128x256
-    {1, {1.529, 1.529}, 6.57, 0.49},  // 192x256
-    {1, {1.852, 1.852}, 8.60, 0.46},  // 256x256
-    {1, {1.720, 1.720}, 9.10, 0.46},  // the five-stage 256x256 kernel (gemm_bf16.hip)
+    {2, {0.203, 0.452}, 2.36, 0.86, 48},  // 32x128
+    {2, {0.190, 0.375}, 2.49, 0.77, 32},  // 64x64
+    {2, {0.325, 0.648}, 2.84, 0.58, 32},  // 64x128
+    {1, {0.639, 0.639}, 3.49, 0.41, 96},  // 64x256
+    {1, {0.585, 0.585}, 3.49, 0.46, 48},  // 128x128
+    {1, {0.740, 0.740}, 5.24, 0.36, 32},  // 192x128
+    {1, {0.945, 0.945}, 5.67, 0.42, 64},  // 128x256
+    {1, {1.529, 1.529}, 6.57, 0.49, 32},  // 192x256
+    {1, {1.852, 1.852}, 8.60, 0.46, 32},  // 256x256
+    {1, {1.720, 1.720}, 9.10, 0.46, 64},  // the five-stage 256x256 kernel (gemm_bf16.hip)
 };
 constexpr double kLaunchUs = 3.9, kReduceUs = 2.2, kReduceBytesPerUs = 10.0e6, kReadBytesPerUs = 5.0e6;
+constexpr double kLargeB = 5.0e7, kLatencyUs = 1.5;
 
 double rounds_us(int t, long long w_total, int kt) {
   const TileCost& c = kCost[t];
@@ -526,7 +529,14 @@ Bf16TilePlan plan_bf16_tiles(uint32_t m, uint32_t n, uint32_t k, bool swiglu) {
         (long long)((m + kTiles[t].bm - 1) / kTiles[t].bm) * ((n + kTiles[t].bn - 1) / kTiles[t].bn);
     for (int s : kSplits) {
       if (s > 1 && (swiglu || all < 3 * s)) break;
-      double us = kLaunchUs + std::max(read_us, rounds_us(t, tiles * s, (all + s - 1) / s));
+      double us = std::max(read_us, rounds_us(t, tiles * s, (all + s - 1) / s));
+      if (2.0 * k * n > kLargeB) {
+        const double readers = (double)std::min<long long>(tiles * s, 256ll * kCost[t].occ) /
+                               ((m + kTiles[t].bm - 1) / kTiles[t].bm);
+        const double rate = std::min(kReadBytesPerUs, readers * kCost[t].flight * 1024.0 / kLatencyUs);
+        us = std::max(us, kCost[t].fill + 2.0 * k * n / rate);
+      }
+      us += kLaunchUs;
       if (s > 1) us += kReduceUs + (double)(s + 1) * m * n * 4.0 / kReduceBytesPerUs;
       if (us < best.us) best = Bf16TilePlan{t, s, us};
     }
