@@ -300,7 +300,9 @@ void build_reference_plan(const PrometheusReductionRequest* r, PrometheusReducti
   p->replay_id = plan_replay_id(p);
 }
 
-// The plan this library executes: one fused dispatch, one wave per row.
+// The plan this library reports for its own execution: one fused stage.  How many
+// waves share a row, and whether a wide row goes over two launches, is the
+// kernels' choice (reduction.hip) and not part of the plan or its replay id.
 void build_executed_plan(uint32_t rows, uint32_t width, uint32_t op, PrometheusReductionPlan* p) {
   memset(p, 0, sizeof(*p));
   p->struct_size = sizeof(*p);
@@ -846,6 +848,7 @@ PROM_REACTOR_API int prometheus_reactor_runtime_reduction_device(void* handle, c
     set_status(out_stage, out_detail_code, PROM_STAGE_INIT, PROM_REDUCTION_DETAIL_RUNTIME_UNAVAILABLE);
     return PROM_ERROR;
   }
+  std::lock_guard<std::mutex> lock(ctx().mu);  // the parts of split rows are runtime-owned
   if (launch_row_reduction(input, output, rows, width, operation, ctx().stream) != hipSuccess) {
     set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_REDUCTION_DETAIL_COMMAND_RECORD_FAILED);
     return PROM_ERROR;
@@ -999,6 +1002,7 @@ PROM_REACTOR_API int prometheus_reactor_runtime_rmsnorm_device(void* handle, con
     set_status(out_stage, out_detail_code, PROM_STAGE_INIT, rt->init_detail);
     return PROM_ERROR;
   }
+  std::lock_guard<std::mutex> lock(ctx().mu);  // the parts of split rows are runtime-owned
   if (launch_rmsnorm(input, weight, output, inv_rms, tokens, width, input_row_stride, epsilon, ctx().stream) !=
       hipSuccess) {
     set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_DETAIL_HIP_LAUNCH_FAILED);

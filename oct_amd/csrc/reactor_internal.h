@@ -62,8 +62,9 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 constexpr uint64_t kRuntimeMagic = 0x4F43544D49333535ull;  // "OCTMI355"
 constexpr uint32_t kEventSlots = 64;
 // Staging slots: 0-3 operand staging, 4 block workspace, 5 block host staging,
-// 6 split-K partials, 7 FFT twiddle table, 8-9 padded GEMM operand copies.
-constexpr uint32_t kStagingSlots = 10;
+// 6 split-K partials, 7 FFT twiddle table, 8-9 padded GEMM operand copies,
+// 10 row-reduction parts.
+constexpr uint32_t kStagingSlots = 11;
 
 struct AsyncState;  // async task table, submission slots and batch arenas (sgemm_async.hip)
 struct ModelState;  // resident model block and compiled session (model_block.hip)
@@ -265,6 +266,7 @@ hipError_t launch_fft64(const double2* in, double2* out, double2* temp, const do
 // Device twiddle table for length n (cached; caller holds ctx().mu): the n/2
 // roots, followed for n > 4096 by the four-step passes' compact tables.
 const double2* fft64_roots(uint32_t n);
+// Row reductions and RMSNorm; the caller holds ctx().mu (staging slot 10).
 hipError_t launch_row_reduction(const float* in, float* out, uint32_t rows, uint32_t width, uint32_t op,
                                 hipStream_t stream);
 // Binary64 reference of the same row reduction (the benchmark's correctness check).

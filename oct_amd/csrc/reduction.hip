@@ -10,21 +10,30 @@
 //
 // MI355X design (the reference's Vulkan path splits a 4096-wide row into
 // 1024-element partial workgroups and runs up to 5 dispatches per softmax,
-// PrometheusReduction.concept:128-164; here every operation is ONE pass):
-//   * one wave64 per row, 4 rows per 256-thread workgroup;
-//   * rows up to 4096 floats with width % 4 == 0 stay in registers: each
-//     lane holds up to 16 float4 (128-bit loads, fully coalesced), so x is
-//     read from HBM exactly once and the output written once;
-//   * cross-lane reductions use wave64 shuffles; sums accumulate in binary64
-//     per lane (free on a bandwidth-bound kernel and closest to the oracle);
-//   * wider or unaligned rows take a streaming variant that re-reads the row
-//     (from L2 for rows that fit) with 32- or 128-bit loads.
+// PrometheusReduction.concept:128-164).  All of it is bound by HBM, so a row is read
+// once and kept in registers, and what varies is how many waves share it:
+//   * one wave per row of at most 1024 values;
+//   * a workgroup of 4 or 16 waves per row of up to 32768 values (one wave per row
+//     left much of the chip idle: RMSNorm of 1056 rows of 3840 values 10.6 us,
+//     four waves per row 7.9; 512 rows of 8192 values, softmax, 87 -> 10.2);
+//   * wider rows over several workgroups of 8192 values each: one
+//     launch leaves each part's sum or (maximum, sum), a second one combines a
+//     row's parts and, for softmax and RMSNorm, reads the row again (from the
+//     caches where it fits) and writes it.  16 rows of 262144 values, softmax:
+//     one wave per row 3165 us, now 17.6.
+// Loads and stores are 16 bytes per lane whatever the row's alignment (4 bytes is
+// enough for them); a width that is not a multiple of 4 ends in single values.
+// Cross-lane steps are wave64 shuffles, cross-wave steps go through LDS; sums
+// accumulate in binary64 (free on a bandwidth-bound kernel and closest to the oracle).
+#include <algorithm>
+
 #include "reactor_internal.h"
 
 namespace prom {
 namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));  // 16 bytes at any float
 
 constexpr uint32_t kOpSum = 1, kOpMax = 2, kOpSoftmax = 3, kOpRms = 4;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -38,6 +47,7 @@ __device__ __forceinline__ double wave_sum_f64(double v) {
   return v;
 }
 
+// `v > m` keeps the oracle's rule: a NaN counts only as the starting value.
 __device__ __forceinline__ float wave_max_f32(float v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -47,198 +57,321 @@ __device__ __forceinline__ float wave_max_f32(float v) {
   return v;
 }
 
-// Register-resident path: width % 4 == 0, width <= 256 * kChunks.  kPreW
-// (RMSNorm of few rows, where each wave's memory latency is the cost): the
-// weight chunks load with the row, before the reduction, instead of after it.
-template <uint32_t kOp, int kChunks, bool kPreW = false>
-__global__ __launch_bounds__(256) void row_resident_kernel(const float* __restrict__ in, const float* __restrict__ w,
-                                                           float* __restrict__ out, float* __restrict__ aux,
-                                                           uint32_t rows, uint32_t width, float eps) {
-  const uint32_t wave = threadIdx.x >> 6;
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t row = blockIdx.x * 4u + wave;
-  if (row >= rows) return;
-  const uint32_t w4 = width >> 2;
-  const floatx4* src = reinterpret_cast<const floatx4*>(in + (size_t)row * width);
+// Sum / maximum over the kWR waves that share a row; every lane gets it.
+template <int kWR>
+__device__ __forceinline__ double row_sum(double v, double* part) {
+  v = wave_sum_f64(v);
+  if constexpr (kWR > 1) {
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = part[0];
+#pragma unroll
+    for (int i = 1; i < kWR; ++i) v += part[i];
+  }
+  return v;
+}
+
+template <int kWR>
+__device__ __forceinline__ float row_max(float v, float* part) {
+  v = wave_max_f32(v);
+  if constexpr (kWR > 1) {
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = v;
+    __syncthreads();
+    v = part[0];
+#pragma unroll
+    for (int i = 1; i < kWR; ++i) v = part[i] > v ? part[i] : v;
+  }
+  return v;
+}
+
+// kThreads threads hold up to 4 * kThreads * kChunks values of a row: thread t has
+// values 4 (c kThreads + t) .. +3 in chunk c.  kTail: the count need not be a
+// multiple of 4.
+template <int kThreads, int kChunks, bool kTail>
+struct RowTile {
   floatx4 v[kChunks];
+
+  static __device__ __forceinline__ uint32_t at(int c, uint32_t t) { return 4u * ((uint32_t)c * kThreads + t); }
+
+  __device__ __forceinline__ void load(const float* __restrict__ src, uint32_t count, uint32_t t) {
 #pragma unroll
-  for (int c = 0; c < kChunks; ++c) {
-    const uint32_t i = (uint32_t)c * 64u + lane;
-    if (i < w4) v[c] = src[i];
+    for (int c = 0; c < kChunks; ++c) {
+      const uint32_t i = at(c, t);
+      if (kTail ? i + 4 <= count : i < count) {
+        v[c] = *reinterpret_cast<const floatx4u*>(src + i);
+      } else if (kTail && i < count) {
+#pragma unroll
+        for (int j = 0; j < 3; ++j) v[c][j] = i + j < count ? src[i + j] : 0.0f;
+      }
+    }
   }
-  if constexpr (kOp == kOpSum) {
-    double acc = 0.0;
+
+  __device__ __forceinline__ void store(float* __restrict__ dst, uint32_t count, uint32_t t) const {
 #pragma unroll
     for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) acc += ((double)v[c].x + (double)v[c].y) + ((double)v[c].z + (double)v[c].w);
-    }
-    acc = wave_sum_f64(acc);
-    if (lane == 0) out[row] = (float)acc;
-  } else if constexpr (kOp == kOpMax) {
-    float m = src[0].x;
+      const uint32_t i = at(c, t);
+      if (kTail ? i + 4 <= count : i < count) {
+        *reinterpret_cast<floatx4u*>(dst + i) = v[c];
+      } else if (kTail && i < count) {
 #pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        m = v[c].x > m ? v[c].x : m;
-        m = v[c].y > m ? v[c].y : m;
-        m = v[c].z > m ? v[c].z : m;
-        m = v[c].w > m ? v[c].w : m;
+        for (int j = 0; j < 3; ++j)
+          if (i + j < count) dst[i + j] = v[c][j];
       }
     }
-    m = wave_max_f32(m);
-    if (lane == 0) out[row] = m;
-  } else if constexpr (kOp == kOpSoftmax) {
-    float m = src[0].x;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        m = v[c].x > m ? v[c].x : m;
-        m = v[c].y > m ? v[c].y : m;
-        m = v[c].z > m ? v[c].z : m;
-        m = v[c].w > m ? v[c].w : m;
-      }
-    }
-    m = wave_max_f32(m);
-    // exp(x - m) = exp2((x - m) * log2 e) on the hardware exp2; the row sum
-    // stays binary64; the normalisation multiplies by one correctly rounded
-    // reciprocal.  Relative error per element is a few fp32 ulps.
-    // (x - m) is formed first: it is exact when x and m are close, so rows of
-    // large nearby values (e.g. 1e4 +- 8) keep full relative accuracy.
-    double acc = 0.0;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        v[c].x = exp2_hw((v[c].x - m) * kLog2e);
-        v[c].y = exp2_hw((v[c].y - m) * kLog2e);
-        v[c].z = exp2_hw((v[c].z - m) * kLog2e);
-        v[c].w = exp2_hw((v[c].w - m) * kLog2e);
-        acc += ((double)v[c].x + (double)v[c].y) + ((double)v[c].z + (double)v[c].w);
-      }
-    }
-    acc = wave_sum_f64(acc);
-    const float rden = (float)(1.0 / acc);
-    floatx4* dst = reinterpret_cast<floatx4*>(out + (size_t)row * width);
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        floatx4 o;
-        o.x = v[c].x * rden;
-        o.y = v[c].y * rden;
-        o.z = v[c].z * rden;
-        o.w = v[c].w * rden;
-        dst[i] = o;
-      }
-    }
-  } else {  // RMSNorm
-    const floatx4* w4p = reinterpret_cast<const floatx4*>(w);
-    floatx4 g[kPreW ? kChunks : 1];
-    if constexpr (kPreW) {
-#pragma unroll
-      for (int c = 0; c < kChunks; ++c) {
-        const uint32_t i = (uint32_t)c * 64u + lane;
-        if (i < w4) g[c] = w4p[i];
-      }
-    }
-    double acc = 0.0;
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        acc += ((double)(v[c].x * v[c].x) + (double)(v[c].y * v[c].y)) +
-               ((double)(v[c].z * v[c].z) + (double)(v[c].w * v[c].w));
-      }
-    }
-    acc = wave_sum_f64(acc);
-    const float sumsq = (float)acc;
-    const float inv = 1.0f / sqrtf(sumsq / (float)width + eps);
-    floatx4* dst = reinterpret_cast<floatx4*>(out + (size_t)row * width);
-#pragma unroll
-    for (int c = 0; c < kChunks; ++c) {
-      const uint32_t i = (uint32_t)c * 64u + lane;
-      if (i < w4) {
-        const floatx4 gc = kPreW ? g[kPreW ? c : 0] : w4p[i];
-        floatx4 o;
-        o.x = v[c].x * inv * gc.x;
-        o.y = v[c].y * inv * gc.y;
-        o.z = v[c].z * inv * gc.z;
-        o.w = v[c].w * inv * gc.w;
-        dst[i] = o;
-      }
-    }
-    if (aux != nullptr && lane == 0) aux[row] = inv;
   }
+
+  // f(value, chunk, element) for every value of the row that this thread holds.
+  template <class F>
+  __device__ __forceinline__ void each(uint32_t count, uint32_t t, F f) {
+#pragma unroll
+    for (int c = 0; c < kChunks; ++c) {
+      const uint32_t i = at(c, t);
+      if (i < count) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (!kTail || j == 0 || i + j < count) f(v[c][j], c, j);
+      }
+    }
+  }
+
+  // The same, replacing each value by f's.
+  template <class F>
+  __device__ __forceinline__ void map(uint32_t count, uint32_t t, F f) {
+    each(count, t, [&](float x, int c, int j) { v[c][j] = f(x, c, j); });
+  }
+
+  __device__ __forceinline__ double sum(uint32_t count, uint32_t t) {
+    double acc = 0.0;
+    if constexpr (kTail) {
+      each(count, t, [&](float x, int, int) { acc += (double)x; });
+    } else {
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c)
+        if (at(c, t) < count) acc += ((double)v[c].x + (double)v[c].y) + ((double)v[c].z + (double)v[c].w);
+    }
+    return acc;
+  }
+
+  __device__ __forceinline__ double sum_squares(uint32_t count, uint32_t t) {
+    double acc = 0.0;
+    if constexpr (kTail) {
+      each(count, t, [&](float x, int, int) { acc += (double)(x * x); });
+    } else {
+#pragma unroll
+      for (int c = 0; c < kChunks; ++c)
+        if (at(c, t) < count)
+          acc += ((double)(v[c].x * v[c].x) + (double)(v[c].y * v[c].y)) +
+                 ((double)(v[c].z * v[c].z) + (double)(v[c].w * v[c].w));
+    }
+    return acc;
+  }
+
+  __device__ __forceinline__ float max(float first, uint32_t count, uint32_t t) {
+    float m = first;
+    each(count, t, [&](float x, int, int) { m = x > m ? x : m; });
+    return m;
+  }
+
+  // Replaces the values by exp(v - m).  (v - m) is formed first: it is exact when
+  // the two are close, so rows of large nearby values (1e4 +- 8) keep full accuracy.
+  // kFast: exp2((v - m) log2 e) on the hardware exp2, a few ulps, for the short
+  // aligned rows; the others use expf.
+  template <bool kFast>
+  __device__ __forceinline__ void exp_minus(float m, uint32_t count, uint32_t t) {
+    map(count, t, [&](float x, int, int) { return kFast ? exp2_hw((x - m) * kLog2e) : expf(x - m); });
+  }
+};
+
+// RMSNorm's scale of a row from its sum of squares.
+__device__ __forceinline__ float inv_rms(double sum, uint32_t width, float eps) {
+  const float sumsq = (float)sum;
+  return 1.0f / sqrtf(sumsq / (float)width + eps);
 }
 
-// Streaming path: any width, any alignment; `stride` is the input row pitch
-// (elements).  Rows are re-read per phase.
-template <uint32_t kOp>
-__global__ __launch_bounds__(256) void row_stream_kernel(const float* __restrict__ in, const float* __restrict__ w,
-                                                         float* __restrict__ out, float* __restrict__ aux,
-                                                         uint32_t rows, uint32_t width, uint32_t stride, float eps) {
-  const uint32_t wave = threadIdx.x >> 6;
-  const uint32_t lane = threadIdx.x & 63;
-  const uint32_t row = blockIdx.x * 4u + wave;
-  if (row >= rows) return;
+// One row per kWR waves (kWR == 1: four rows per workgroup), width at most
+// 256 kWR kChunks.  RMSNorm's weights load with the row: with few rows each wave's
+// memory latency is the cost.
+template <uint32_t kOp, int kWR, int kChunks, bool kTail>
+__global__ __launch_bounds__(kWR == 1 ? 256 : 64 * kWR) void row_kernel(const float* __restrict__ in,
+                                                                        const float* __restrict__ w,
+                                                                        float* __restrict__ out,
+                                                                        float* __restrict__ aux, uint32_t rows,
+                                                                        uint32_t width, uint32_t stride, float eps) {
+  constexpr int kThreads = 64 * kWR;
+  constexpr bool kFast = !kTail && kWR * kChunks <= 16;
+  __shared__ double part_d[kWR];
+  __shared__ float part_f[kWR];
+  const uint32_t t = kWR == 1 ? threadIdx.x & 63 : threadIdx.x;
+  const uint32_t row = kWR == 1 ? blockIdx.x * 4u + (threadIdx.x >> 6) : blockIdx.x;
+  if (kWR == 1 && row >= rows) return;
   const float* src = in + (size_t)row * stride;
+  RowTile<kThreads, kChunks, kTail> x;
+  x.load(src, width, t);
   if constexpr (kOp == kOpSum) {
-    double acc = 0.0;
-    for (uint32_t i = lane; i < width; i += 64) acc += (double)src[i];
-    acc = wave_sum_f64(acc);
-    if (lane == 0) out[row] = (float)acc;
+    const double s = row_sum<kWR>(x.sum(width, t), part_d);
+    if (t == 0) out[row] = (float)s;
   } else if constexpr (kOp == kOpMax) {
-    float m = src[0];
-    for (uint32_t i = lane; i < width; i += 64) m = src[i] > m ? src[i] : m;
-    m = wave_max_f32(m);
-    if (lane == 0) out[row] = m;
+    const float m = row_max<kWR>(x.max(src[0], width, t), part_f);
+    if (t == 0) out[row] = m;
   } else if constexpr (kOp == kOpSoftmax) {
-    float m = src[0];
-    for (uint32_t i = lane; i < width; i += 64) m = src[i] > m ? src[i] : m;
-    m = wave_max_f32(m);
-    double acc = 0.0;
-    for (uint32_t i = lane; i < width; i += 64) acc += (double)expf(src[i] - m);
-    acc = wave_sum_f64(acc);
-    const float denom = (float)acc;
-    float* dst = out + (size_t)row * width;
-    for (uint32_t i = lane; i < width; i += 64) dst[i] = expf(src[i] - m) / denom;
+    const float m = row_max<kWR>(x.max(src[0], width, t), part_f);
+    x.template exp_minus<kFast>(m, width, t);
+    const double s = row_sum<kWR>(x.sum(width, t), part_d);
+    const float rden = (float)(1.0 / s);  // one correctly rounded reciprocal
+    x.map(width, t, [&](float y, int, int) { return y * rden; });
+    x.store(out + (size_t)row * width, width, t);
   } else {
-    double acc = 0.0;
-    for (uint32_t i = lane; i < width; i += 64) acc += (double)(src[i] * src[i]);
-    acc = wave_sum_f64(acc);
-    const float sumsq = (float)acc;
-    const float inv = 1.0f / sqrtf(sumsq / (float)width + eps);
-    float* dst = out + (size_t)row * width;
-    for (uint32_t i = lane; i < width; i += 64) dst[i] = src[i] * inv * w[i];
-    if (aux != nullptr && lane == 0) aux[row] = inv;
+    RowTile<kThreads, kChunks, kTail> g;
+    g.load(w, width, t);
+    const float inv = inv_rms(row_sum<kWR>(x.sum_squares(width, t), part_d), width, eps);
+    x.map(width, t, [&](float y, int c, int j) { return y * inv * g.v[c][j]; });
+    x.store(out + (size_t)row * width, width, t);
+    if (aux != nullptr && t == 0) aux[row] = inv;
   }
 }
 
+// Rows over several workgroups: part p of a row is its values [8192 p, 8192 p +
+// 8192).  parts[row * n + p] is the part's sum (sum, RMSNorm: of squares), maximum
+// (in `max`), or both: (maximum, sum of exp(x - maximum)).
+constexpr uint32_t kPartValues = 8192;
+
+struct RowPart {
+  double sum;
+  float max;
+  float pad;
+};
+
+template <uint32_t kOp>
+__global__ __launch_bounds__(256) void row_parts_kernel(const float* __restrict__ in, RowPart* __restrict__ parts,
+                                                        uint32_t n, uint32_t width, uint32_t stride) {
+  __shared__ double part_d[4];
+  __shared__ float part_f[4];
+  const uint32_t row = blockIdx.x / n, p = blockIdx.x - row * n, t = threadIdx.x;
+  const float* src = in + (size_t)row * stride;
+  const uint32_t count = min(kPartValues, width - p * kPartValues);
+  RowTile<256, 8, true> x;
+  x.load(src + p * kPartValues, count, t);
+  RowPart r{0.0, 0.0f, 0.0f};
+  if constexpr (kOp == kOpMax || kOp == kOpSoftmax) r.max = row_max<4>(x.max(src[0], count, t), part_f);
+  if constexpr (kOp == kOpSoftmax) {
+    // A part of negative infinities alone adds nothing (and NaN where the whole
+    // row is that): its sum is finite and gets the factor exp(-inf - maximum).
+    x.template exp_minus<false>(r.max == -__builtin_inff() ? 0.0f : r.max, count, t);
+  }
+  if constexpr (kOp == kOpSum || kOp == kOpSoftmax) r.sum = row_sum<4>(x.sum(count, t), part_d);
+  if constexpr (kOp == kOpRms) r.sum = row_sum<4>(x.sum_squares(count, t), part_d);
+  if (t == 0) parts[blockIdx.x] = r;
+}
+
+// Combines the n parts of a row in every wave, lane l taking parts l, l + 64, ...
+template <uint32_t kOp>
+__device__ __forceinline__ RowPart combine_parts(const RowPart* __restrict__ parts, uint32_t n) {
+  const uint32_t lane = threadIdx.x & 63;
+  RowPart r{0.0, parts[0].max, 0.0f};
+  if constexpr (kOp == kOpMax || kOp == kOpSoftmax) {
+    for (uint32_t i = lane; i < n; i += 64) r.max = parts[i].max > r.max ? parts[i].max : r.max;
+    r.max = wave_max_f32(r.max);
+  }
+  if constexpr (kOp != kOpMax) {
+    for (uint32_t i = lane; i < n; i += 64)
+      r.sum += kOp == kOpSoftmax ? parts[i].sum * exp((double)parts[i].max - (double)r.max) : parts[i].sum;
+    r.sum = wave_sum_f64(r.sum);
+  }
+  return r;
+}
+
+// Sum and max: a wave per row.  Softmax and RMSNorm: a workgroup per part.
+template <uint32_t kOp>
+__global__ __launch_bounds__(256) void row_finish_kernel(const float* __restrict__ in, const float* __restrict__ w,
+                                                         float* __restrict__ out, float* __restrict__ aux,
+                                                         const RowPart* __restrict__ parts, uint32_t n, uint32_t rows,
+                                                         uint32_t width, uint32_t stride, float eps) {
+  if constexpr (kOp == kOpSum || kOp == kOpMax) {
+    const uint32_t row = blockIdx.x * 4u + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const RowPart r = combine_parts<kOp>(parts + (size_t)row * n, n);
+    if ((threadIdx.x & 63) == 0) out[row] = kOp == kOpSum ? (float)r.sum : r.max;
+  } else {
+    const uint32_t row = blockIdx.x / n, p = blockIdx.x - row * n, t = threadIdx.x;
+    const uint32_t count = min(kPartValues, width - p * kPartValues);
+    RowTile<256, 8, true> x;
+    x.load(in + (size_t)row * stride + p * kPartValues, count, t);
+    const RowPart r = combine_parts<kOp>(parts + (size_t)row * n, n);
+    if constexpr (kOp == kOpSoftmax) {
+      const float rden = (float)(1.0 / r.sum);
+      x.template exp_minus<false>(r.max, count, t);
+      x.map(count, t, [&](float y, int, int) { return y * rden; });
+    } else {
+      const float inv = inv_rms(r.sum, width, eps);
+      RowTile<256, 8, true> g;
+      g.load(w + p * kPartValues, count, t);
+      x.map(count, t, [&](float y, int c, int j) { return y * inv * g.v[c][j]; });
+      if (aux != nullptr && p == 0 && t == 0) aux[row] = inv;
+    }
+    x.store(out + (size_t)row * width + p * kPartValues, count, t);
+  }
+}
+
+// How a call runs: `waves` per row holding `chunks` chunks each, or split rows.
+// us at 6 TB/s would be 44.7 for softmax of 8192 rows of 4096: one wave of 16
+// chunks 52.1, four of 4 48.6; 4096 rows of 8192: four waves of 8 51.9, sixteen of 4
+// 49.4, and sums 23.4 and 24.4 the other way round; 8192 rows of 1000: one wave
+// 11.5, four 12.9.  Rows of up to 32768 stay whole while there are enough of them
+// (softmax of 1024 rows of 32768: whole 65, split 84; 256 rows: 16.6 and 23.6).
+struct RowPlan {
+  int waves, chunks;  // waves 0: rows over several workgroups
+};
+
+RowPlan plan_rows(uint32_t op, uint32_t rows, uint32_t width) {
+  if (width > 32768u || (width > kPartValues && rows <= 32u)) return {0, 0};
+  if (width <= 1024u) return {1, width <= 256u ? 1 : 4};
+  if (width <= 4096u) return {4, width <= 2048u ? 2 : 4};
+  if (width <= 8192u && (op == kOpSum || op == kOpMax)) return {4, 8};
+  return {16, width <= 16384u ? 4 : 8};
+}
+
+template <uint32_t kOp, bool kTail>
+hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, float* aux, uint32_t rows,
+                       uint32_t width, uint32_t stride, float eps, hipStream_t stream) {
+  if (p.waves == 0) {
+    const uint32_t n = (width + kPartValues - 1) / kPartValues;
+    RowPart* parts = static_cast<RowPart*>(staging(10, (size_t)rows * n * sizeof(RowPart)));
+    if (parts == nullptr) return hipErrorOutOfMemory;
+    hipLaunchKernelGGL((row_parts_kernel<kOp>), dim3(rows * n), dim3(256), 0, stream, in, parts, n, width, stride);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    const uint32_t blocks = kOp == kOpSum || kOp == kOpMax ? (rows + 3u) / 4u : rows * n;
+    hipLaunchKernelGGL((row_finish_kernel<kOp>), dim3(blocks), dim3(256), 0, stream, in, w, out, aux, parts, n, rows,
+                       width, stride, eps);
+    return hipGetLastError();
+  }
+#define ROWS(W, C)                                                                                                   \
+  hipLaunchKernelGGL((row_kernel<kOp, W, C, kTail>), dim3(W == 1 ? (rows + 3u) / 4u : rows),                         \
+                     dim3(W == 1 ? 256 : 64 * W), 0, stream, in, w, out, aux, rows, width, stride, eps);             \
+  break
+  switch (p.waves * 100 + p.chunks) {
+    case 101: ROWS(1, 1);
+    case 104: ROWS(1, 4);
+    case 402: ROWS(4, 2);
+    case 404: ROWS(4, 4);
+    case 408: ROWS(4, 8);
+    case 1604: ROWS(16, 4);
+    case 1608: ROWS(16, 8);
+    default: return hipErrorInvalidValue;
+  }
+#undef ROWS
+  return hipGetLastError();
+}
+
+// Rows of whole 16-byte chunks at 16-byte addresses take the kernels without tails.
 template <uint32_t kOp>
 hipError_t dispatch(const float* in, const float* w, float* out, float* aux, uint32_t rows, uint32_t width,
                     uint32_t stride, float eps, hipStream_t stream) {
-  const dim3 grid((rows + 3u) / 4u);
-  const dim3 block(256);
-  const bool resident = (width % 4u == 0u) && (stride == width) && ((reinterpret_cast<uintptr_t>(in) & 15u) == 0) &&
-                        ((reinterpret_cast<uintptr_t>(out) & 15u) == 0) &&
-                        (w == nullptr || (reinterpret_cast<uintptr_t>(w) & 15u) == 0);
-  if (resident && width <= 256u * 4u) {
-    hipLaunchKernelGGL((row_resident_kernel<kOp, 4>), grid, block, 0, stream, in, w, out, aux, rows, width, eps);
-  } else if (resident && width <= 256u * 16u) {
-    // Few rows (a transformer layer's tokens): one wave per row leaves the
-    // chip mostly idle, so each wave's latency is the cost; preload the weights.
-    if (kOp == kOpRms && rows <= 2048u && width <= 256u * 8u)
-      hipLaunchKernelGGL((row_resident_kernel<kOp, 8, true>), grid, block, 0, stream, in, w, out, aux, rows, width,
-                         eps);
-    else
-      hipLaunchKernelGGL((row_resident_kernel<kOp, 16>), grid, block, 0, stream, in, w, out, aux, rows, width, eps);
-  } else {
-    hipLaunchKernelGGL((row_stream_kernel<kOp>), grid, block, 0, stream, in, w, out, aux, rows, width, stride, eps);
-  }
-  return hipGetLastError();
+  const RowPlan p = plan_rows(kOp, rows, width);
+  const bool whole = width % 4u == 0 && stride == width && (reinterpret_cast<uintptr_t>(in) & 15u) == 0 &&
+                     (reinterpret_cast<uintptr_t>(out) & 15u) == 0 && (reinterpret_cast<uintptr_t>(w) & 15u) == 0;
+  return whole ? launch_rows<kOp, false>(p, in, w, out, aux, rows, width, stride, eps, stream)
+               : launch_rows<kOp, true>(p, in, w, out, aux, rows, width, stride, eps, stream);
 }
 
 // The benchmark entry's correctness reference: the same reduction with every
