@@ -169,11 +169,27 @@ hipError_t launch_sgemm_f32_unreduced(const float* a, int lda, const float* b, i
                                       int max_slices, hipStream_t stream, int* slices);
 // The slices launch_sgemm_f32_unreduced leaves for 16-byte aligned operands (1: none).
 int sgemm_f32_unreduced_slices(int lda, int ldb, uint32_t m, uint32_t n, uint32_t k, int max_slices);
+// Products of at most 48 rows (sgemm_rows.hip): plan_sgemm_rows picks the workgroup
+// shape and the K slices with the least estimated time, launch_sgemm_rows runs it;
+// with splits > 1 c takes the slices, m * ldc floats apart, and the caller adds
+// them.  The geglu form is launch_sgemm_f32_geglu's product, never sliced.
+struct SgemmRowsPlan {
+  int shape, splits;
+  double us;
+};
+bool sgemm_rows_take(uint32_t m, uint32_t k, int lda, int ldb, int halves);
+SgemmRowsPlan plan_sgemm_rows(uint32_t m, uint32_t n, uint32_t k, bool geglu, uint64_t max_partial_floats);
+int sgemm_rows_columns(const SgemmRowsPlan& plan);
+hipError_t launch_sgemm_rows(const SgemmRowsPlan& plan, const float* a, int lda, const float* b, int ldb, float* c,
+                             int ldc, uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr,
+                             hipStream_t stream);
+hipError_t launch_sgemm_rows_geglu(const SgemmRowsPlan& plan, const float* a, int lda, const float* w, float* h,
+                                   int ldh, uint32_t m, uint32_t f, uint32_t k, hipStream_t stream);
 // H[m, f] = gelu_tanh(A @ W[:, :f]) * (A @ W[:, f:]) for W = [gate | up]
-// ([k, 2f], row pitch 2f): one launch of the 128x128 direct-to-LDS kernel
-// whose tiles take 64 gate and the matching 64 up columns.  Returns
-// hipErrorNotSupported when the shape does not fit it (f % 64, k % 16,
-// 16-byte aligned operands and rows, byte offsets below 2^31); the caller
+// ([k, 2f], row pitch 2f): one launch, of the few-rows kernel or of the 128x128
+// direct-to-LDS kernel whose tiles take 64 gate and the matching 64 up columns.
+// Returns hipErrorNotSupported when the shape fits neither (the tiles: f % 64, k %
+// 16, 16-byte aligned operands and rows, byte offsets below 2^31); the caller
 // then runs the GEMM and the elementwise GeGLU.
 hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float* h, int ldh, uint32_t m, uint32_t f,
                                   uint32_t k, hipStream_t stream);

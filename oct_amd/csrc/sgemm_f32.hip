@@ -1091,6 +1091,25 @@ void launch_tile(bool buf, bool vec, dim3 grid, hipStream_t stream, const float*
                        tiles_m, tiles_n, lda, ldb, ldc, r, ldr, k_len, sa, sb, sc);
 }
 
+// c = the sum of `splits` slices of partial (m * n floats apart) + residual.
+hipError_t launch_splitk_reduce(const float* partial, float* c, uint32_t m, uint32_t n, int ldc, int splits,
+                                const float* residual, int ldr, hipStream_t stream) {
+  const bool vec4 = n % 4 == 0 && ldc % 4 == 0 && aligned16(c) &&
+                    (residual == nullptr || (ldr % 4 == 0 && aligned16(residual)));
+  if (vec4 && splits <= 16) {
+    const unsigned bx = (unsigned)((n / 4 + 255) / 256);
+    const unsigned by = (unsigned)std::min<uint32_t>(m, std::max(1u, 8192u / bx));
+    hipLaunchKernelGGL(splitk_reduce4_kernel, dim3(bx, by), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
+                       splits, residual, ldr);
+  } else {
+    const size_t total = (size_t)m * n;
+    const unsigned blocks = (unsigned)std::min((size_t)8192, (total + 255) / 256);
+    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
+                       splits, residual, ldr);
+  }
+  return hipGetLastError();
+}
+
 // Launches the MFMA kernel of plan p over `batch` matrices (batch > 1 only
 // without split) and, when split, the reduce into c (partial: splits*m*n floats).
 hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long sa, const float* b, int ldb,
@@ -1153,31 +1172,19 @@ hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long
                            ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
   }
-  if (split && reduce) {
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const bool vec4 = n % 4 == 0 && ldc % 4 == 0 && aligned16(c) && (residual == nullptr || (ldr % 4 == 0 && aligned16(residual)));
-    if (vec4 && p.splits <= 16) {
-      const unsigned bx = (unsigned)((n / 4 + 255) / 256);
-      const unsigned by = (unsigned)std::min<uint32_t>(m, std::max(1u, 8192u / bx));
-      hipLaunchKernelGGL(splitk_reduce4_kernel, dim3(bx, by), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
-                         p.splits, residual, ldr);
-    } else {
-      const size_t total = (size_t)m * n;
-      const unsigned blocks = (unsigned)std::min((size_t)8192, (total + 255) / 256);
-      hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
-                         p.splits, residual, ldr);
-    }
-  }
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess || !split || !reduce) return e;
+  return launch_splitk_reduce(partial, c, m, n, ldc, p.splits, residual, ldr, stream);
 }
 
-// What launch_sgemm_f32_ex queues for one product: the GEMV, or one or two
-// MFMA products (rows [0, head_rows) and, after a tail split, the rest),
-// optionally on padded copies of A and B.  A pure function of the shape,
+// What launch_sgemm_f32_ex queues for one product: the GEMV, the few-rows kernel
+// (sgemm_rows.hip), or one or two MFMA products (rows [0, head_rows) and, after a
+// tail split, the rest), optionally on padded copies of A and B.  A pure function of the shape,
 // strides and operand alignment.
 struct SgemmSchedule {
   bool gemv;
+  bool few_rows;
+  SgemmRowsPlan rows;  // few_rows
   bool tail_split;
   bool repack;         // A, B copied first to [m][k4] and [k4][n4], 16-byte rows, zero padding
   uint32_t k4, n4;     // padded K and B row stride when repacking
@@ -1242,8 +1249,23 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
         r.repack = true;
         r.k4 = k4;
         r.n4 = n4;
-        return r;
+        s = r;
       }
+    }
+  }
+  if (sgemm_rows_take(m, k, lda, ldb, 1)) {
+    const SgemmRowsPlan rows = plan_sgemm_rows(m, n, k, false, max_partial_floats);
+    // The two models meet where both are off: a sliced product of a small B measured
+    // slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger one faster
+    // (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
+    const bool small = (uint64_t)n * k < (1u << 20);
+    const double bias = small ? (rows.splits > 1 ? 1.2 : 0.0) : -0.06 * s.cost_us;
+    if (rows.us + bias < s.cost_us) {
+      s = SgemmSchedule{};
+      s.few_rows = true;
+      s.rows = rows;
+      s.head_rows = m;
+      s.cost_us = rows.us;
     }
   }
   return s;
@@ -1258,7 +1280,7 @@ uint64_t schedule_repack_floats(const SgemmSchedule& s, uint32_t m) {
 // and 9) receives the padded copies of a repacking schedule, A then B.
 hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, const float* b, int ldb, float* c,
                               int ldc, uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr,
-                              float* partial, float* packed, hipStream_t stream) {
+                              float* partial, float* packed, hipStream_t stream, bool reduce = true) {
   if (s.gemv) {
     const bool vec = (k % 4 == 0) && aligned16(a) && aligned16(b);
     const dim3 grid((m + 3) / 4);
@@ -1267,6 +1289,18 @@ hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, c
     else
       hipLaunchKernelGGL(gemv_f32_kernel<false>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)k);
     return hipGetLastError();
+  }
+  if (s.few_rows) {
+    SgemmRowsPlan p = s.rows;
+    float* part = nullptr;
+    if (p.splits > 1) {
+      part = partial != nullptr ? partial : static_cast<float*>(staging(6, (size_t)p.splits * m * n * sizeof(float)));
+      if (part == nullptr) p.splits = 1;
+    }
+    if (p.splits == 1) return launch_sgemm_rows(p, a, lda, b, ldb, c, ldc, m, n, k, residual, ldr, stream);
+    const hipError_t e = launch_sgemm_rows(p, a, lda, b, ldb, part, (int)n, m, n, k, nullptr, 0, stream);
+    if (e != hipSuccess || !reduce) return e;
+    return launch_splitk_reduce(part, c, m, n, ldc, p.splits, residual, ldr, stream);
   }
   if (s.repack) {
     float* pa = packed != nullptr ? packed : static_cast<float*>(staging(8, (size_t)m * s.k4 * sizeof(float)));
@@ -1305,6 +1339,7 @@ hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, c
 
 uint64_t schedule_partial_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
   if (s.gemv) return 0;
+  if (s.few_rows) return s.rows.splits > 1 ? (uint64_t)s.rows.splits * m * n : 0;
   uint64_t need = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * s.head_rows * n : 0;
   if (s.tail_split && s.plan[1].splits > 1)
     need = std::max<uint64_t>(need, (uint64_t)s.plan[1].splits * (m - s.head_rows) * n);
@@ -1328,10 +1363,15 @@ hipError_t launch_sgemm_f32_ex(const float* a, int lda, const float* b, int ldb,
   return run_sgemm_schedule(s, a, lda, b, ldb, c, ldc, m, n, k, residual, ldr, nullptr, nullptr, stream);
 }
 
+// K slices of a schedule that is one sliced product (1: it is not).
+static int schedule_slices(const SgemmSchedule& s) {
+  if (s.gemv || s.repack || s.tail_split) return 1;
+  return s.few_rows ? s.rows.splits : s.plan[0].splits;
+}
+
 int sgemm_f32_unreduced_slices(int lda, int ldb, uint32_t m, uint32_t n, uint32_t k, int max_slices) {
-  const SgemmSchedule s = schedule_sgemm(true, lda, ldb, m, n, k, false, ~0ull);
-  if (s.gemv || s.repack || s.tail_split || s.plan[0].splits <= 1 || s.plan[0].splits > max_slices) return 1;
-  return s.plan[0].splits;
+  const int slices = schedule_slices(schedule_sgemm(true, lda, ldb, m, n, k, false, ~0ull));
+  return slices > max_slices ? 1 : slices;
 }
 
 hipError_t launch_sgemm_f32_unreduced(const float* a, int lda, const float* b, int ldb, float* c, int ldc,
@@ -1339,10 +1379,12 @@ hipError_t launch_sgemm_f32_unreduced(const float* a, int lda, const float* b, i
                                       int max_slices, hipStream_t stream, int* slices) {
   *slices = 1;
   const SgemmSchedule s = schedule_sgemm(aligned16(a) && aligned16(b), lda, ldb, m, n, k, false, ~0ull);
-  if (s.gemv || s.repack || s.tail_split || s.plan[0].splits <= 1 || s.plan[0].splits > max_slices ||
-      partial == nullptr || (uint64_t)s.plan[0].splits * m * n > partial_floats)
+  const int cut = schedule_slices(s);
+  if (cut <= 1 || cut > max_slices || partial == nullptr || (uint64_t)cut * m * n > partial_floats)
     return run_sgemm_schedule(s, a, lda, b, ldb, c, ldc, m, n, k, nullptr, 0, nullptr, nullptr, stream);
-  *slices = s.plan[0].splits;
+  *slices = cut;
+  if (s.few_rows)
+    return run_sgemm_schedule(s, a, lda, b, ldb, c, ldc, m, n, k, nullptr, 0, partial, nullptr, stream, false);
   return run_sgemm_plan(s.plan[0], a, lda, 0, b, ldb, 0, c, ldc, 0, m, n, k, 1, nullptr, 0, partial, stream,
                         false);
 }
@@ -1398,6 +1440,13 @@ hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float
                                   uint32_t k, hipStream_t stream) {
   if (m == 0 || f == 0 || k == 0) return hipErrorNotSupported;
   const int ldb = (int)(2 * f);
+  // Few rows: the tiles would run most of theirs as padding (15 rows of the Gemma
+  // layer's 2048 x 2 * 16384: 132 us).
+  if (sgemm_rows_take(m, k, lda, ldb, 2)) {
+    const SgemmRowsPlan rows = plan_sgemm_rows(m, f, k, true, 0);
+    const double tiles = plan_cost(SgemmPlan{4, 1, (int)k}, m, 2 * f, 1);
+    if (rows.us < tiles) return launch_sgemm_rows_geglu(rows, a, lda, w, h, ldh, m, f, k, stream);
+  }
   const bool ok = f % 64 == 0 && buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k, (int)k, 4) &&
                   ldh % 4 == 0 && aligned16(h);
   if (!ok) return hipErrorNotSupported;
@@ -1466,6 +1515,19 @@ extern "C" PROM_REACTOR_API int prometheus_reactor_sgemm_plan(uint32_t m, uint32
     return PROM_OK;
   }
   out_plan->detail_code = PROM_DETAIL_PATH_HIP_MFMA_F32;
+  out_plan->estimated_us = s.cost_us;
+  if (s.few_rows) {
+    out_plan->products = 1u;
+    out_plan->tile_m[0] = (m + 15u) / 16u * 16u;
+    out_plan->tile_n[0] = (uint32_t)sgemm_rows_columns(s.rows);
+    out_plan->k_slices[0] = (uint32_t)s.rows.splits;
+    out_plan->k_slice_len[0] = (k + 15u) / 16u / (uint32_t)s.rows.splits * 16u;
+    if (s.rows.splits == 1) out_plan->k_slice_len[0] = k;
+    out_plan->launches = s.rows.splits > 1 ? 2u : 1u;
+    out_plan->partial_bytes = schedule_partial_floats(s, m, n) * sizeof(float);
+    if (has_scratch) out_plan->scratch_bytes = schedule_scratch_floats(s, m, n) * sizeof(float);
+    return PROM_OK;
+  }
   out_plan->products = s.tail_split ? 2u : 1u;
   out_plan->repacked = s.repack ? 1u : 0u;
   out_plan->repack_bytes = schedule_repack_floats(s, m) * sizeof(float);
@@ -1485,7 +1547,6 @@ extern "C" PROM_REACTOR_API int prometheus_reactor_sgemm_plan(uint32_t m, uint32
   }
   if (s.repack) out_plan->launches += 2u;
   out_plan->partial_bytes = schedule_partial_floats(s, m, n) * sizeof(float);
-  out_plan->estimated_us = s.cost_us;
   if (has_scratch) out_plan->scratch_bytes = schedule_scratch_floats(s, m, n) * sizeof(float);
   return PROM_OK;
 }
