@@ -285,10 +285,10 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
 // one 128-bit read, so step (p, j) pairs k = 8p + j (lanes 0-31) with
 // k = 8p + 4 + j (lanes 32-63); the B operand reads the same two k rows.
 // Every k of the tile enters each accumulator exactly once.
-template <int kBN>
+template <int kBN, int kBM = 128>
 struct DlCfg {
   static constexpr int kNI = kBN / 64;
-  static constexpr int kABytes = 128 * kBK * 4;
+  static constexpr int kABytes = kBM * kBK * 4;
   static constexpr int kBPitch = kBN == 256 ? 1056 : 512;
   static constexpr int kStage = kABytes + kBK * kBPitch;
 };
@@ -299,18 +299,22 @@ struct DlCfg {
 // are a gate block and its up block (tile columns 0-31 gate, 32-63 up, 64-95
 // gate + 32, 96-127 up + 32); the epilogue stores gelu_tanh(gate) * up, N
 // columns in all.
-template <int kBN, int kWaves, bool kGeGLU = false>
+template <int kBN, int kBM, bool kGeGLU = false>
 __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, const float* __restrict__ B, float* C,
                                                   int M, int N, int K, int tiles_m, int tiles_n, int lda, int ldb,
                                                   int ldc, const float* R, int ldr, int k_len, long long sa,
                                                   long long sb, long long sc, char* S0, char* S1) {
-  static_assert(!kGeGLU || (kBN == 128 && kWaves == 8), "the GeGLU tile is the eight-wave 128x128 one");
-  using D = DlCfg<kBN>;
+  static_assert(!kGeGLU || kBN == 128, "the GeGLU tiles are 128 wide");
+  static_assert(kBN == 128 || kBM == 128, "the 256-wide tile has 128 rows");
+  using D = DlCfg<kBN, kBM>;
   constexpr int kNI = D::kNI;
-  constexpr int kRW = 256 / kWaves;                  // rows per wave (waves: kWaves/2 along M, 2 along N)
+  constexpr int kRW = kBN == 256 ? 64 : 32;  // rows per wave (two waves along N)
+  constexpr int kWaves = 2 * kBM / kRW;
   constexpr int kMI = kRW / 32;
-  constexpr int kAI = 8 / kWaves;                    // A transfers (16-row blocks) per wave
-  constexpr int kBI = (kBN == 256 ? 16 : 8) / kWaves;  // B transfers per wave
+  constexpr int kABlocks = kBM / 16, kBBlocks = kBN == 256 ? 16 : 8;  // 1 KB transfers per K tile
+  constexpr int kAI = kABlocks / kWaves;
+  constexpr int kBI = (kBBlocks + kWaves - 1) / kWaves;
+  static_assert(kABlocks == kAI * kWaves, "whole A transfers per wave");
   typedef __attribute__((address_space(3))) void lds_void;
 
   if (gridDim.z > 1) {
@@ -320,7 +324,7 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
   }
   int tm, tn;
   map_tile(tiles_m, tiles_n, &tm, &tn);
-  const int row0 = tm * 128;
+  const int row0 = tm * kBM;
   const int col0 = kGeGLU ? tn * (kBN / 2) : tn * kBN;
   size_t a_extent = (size_t)M * lda;
   if (gridDim.y > 1) {
@@ -355,10 +359,10 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
 #pragma unroll
   for (int i = 0; i < kBI; ++i) {
     if constexpr (kBN == 256) {
-      const int kr = kBI * wave + i;  // one 256-wide row per instruction
+      const int kr = i * kWaves + wave;  // one 256-wide row per instruction
       b_off[i] = (uint32_t)((kr * ldb + col0 + 4 * lane) * 4);
     } else {
-      const int q = kBI * wave + i;  // rows 2q, 2q+1
+      const int q = i * kWaves + wave;  // rows 2q, 2q+1
       const int kr = 2 * q + (lane >> 5);
       const int c = (lane & 31) ^ (((kr >> 2) & 1) << 3);
       int gcol = col0 + 4 * c;
@@ -378,8 +382,9 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
                                                0, 0);
 #pragma unroll
     for (int i = 0; i < kBI; ++i) {
-      char* dst = kBN == 256 ? stage + D::kABytes + (kBI * wave + i) * D::kBPitch
-                             : stage + D::kABytes + (kBI * wave + i) * 1024;
+      const int q = i * kWaves + wave;
+      if (kBBlocks % kWaves != 0 && q >= kBBlocks) break;  // fewer blocks than waves, or a remainder
+      char* dst = stage + D::kABytes + q * (kBN == 256 ? D::kBPitch : 1024);
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rsb, (lds_void*)dst, 16, b_off[i], sb_k, 0, 0);
     }
   };
@@ -499,7 +504,7 @@ __global__ __launch_bounds__(256, 3) void sgemm_f32_dl256_kernel(const float* __
                                                                  long long sa, long long sb, long long sc) {
   __shared__ __attribute__((aligned(1024))) char S0[DlCfg<256>::kStage];
   __shared__ __attribute__((aligned(1024))) char S1[DlCfg<256>::kStage];
-  sgemm_f32_dl_body<256, 4>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
+  sgemm_f32_dl_body<256, 128>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
 }
 
 // 128x128 with eight waves (each 32x64, 50 VGPRs): two waves per SIMD even
@@ -516,19 +521,36 @@ __global__ __launch_bounds__(512, 1) void sgemm_f32_dl128w8_kernel(const float* 
                                                                    long long sc) {
   __shared__ __attribute__((aligned(1024))) char S0[DlCfg<128>::kStage];
   __shared__ __attribute__((aligned(1024))) char S1[DlCfg<128>::kStage];
-  sgemm_f32_dl_body<128, 8>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
+  sgemm_f32_dl_body<128, 128>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
+}
+
+// The same with 64 rows (four waves of 32x64), for row counts that 128 divides
+// badly: 1056x11520x3840 669 us, the 64x64 tile 697, 128x128 with a tail 728.
+// (Heights of 96, 160, 192, 224 and 256 rows were the fastest tile of none of 53
+// shapes: with 6, 10 or 14 waves the SIMDs' shares are uneven.)
+__global__ __launch_bounds__(256, 1) void sgemm_f32_dl64x128_kernel(const float* __restrict__ A,
+                                                                    const float* __restrict__ B, float* C, int M,
+                                                                    int N, int K, int tiles_m, int tiles_n, int lda,
+                                                                    int ldb, int ldc, const float* R, int ldr,
+                                                                    int k_len, long long sa, long long sb,
+                                                                    long long sc) {
+  __shared__ __attribute__((aligned(1024))) char S0[DlCfg<128, 64>::kStage];
+  __shared__ __attribute__((aligned(1024))) char S1[DlCfg<128, 64>::kStage];
+  sgemm_f32_dl_body<128, 64>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
 }
 
 // The gate|up product of the Gemma-style layer with GeGLU in the epilogue
-// (sgemm_f32_dl_body's kGeGLU): C is the [M, N] GeGLU output.
-__global__ __launch_bounds__(512, 1) void sgemm_f32_dl128w8_geglu_kernel(const float* __restrict__ A,
-                                                                         const float* __restrict__ B, float* C,
-                                                                         int M, int N, int K, int tiles_m,
-                                                                         int tiles_n, int lda, int ldb, int ldc) {
-  __shared__ __attribute__((aligned(1024))) char S0[DlCfg<128>::kStage];
-  __shared__ __attribute__((aligned(1024))) char S1[DlCfg<128>::kStage];
-  sgemm_f32_dl_body<128, 8, true>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, nullptr, 0, K, 0, 0, 0, S0,
-                                  S1);
+// (sgemm_f32_dl_body's kGeGLU): C is the [M, N] GeGLU output.  64, 128 or 192 rows
+// per tile (geglu_height).
+template <int kBM>
+__global__ __launch_bounds__(4 * kBM, 1) void sgemm_f32_dl128h_geglu_kernel(const float* __restrict__ A,
+                                                                            const float* __restrict__ B, float* C,
+                                                                            int M, int N, int K, int tiles_m,
+                                                                            int tiles_n, int lda, int ldb, int ldc) {
+  __shared__ __attribute__((aligned(1024))) char S0[DlCfg<128, kBM>::kStage];
+  __shared__ __attribute__((aligned(1024))) char S1[DlCfg<128, kBM>::kStage];
+  sgemm_f32_dl_body<128, kBM, true>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, nullptr, 0, K, 0, 0, 0, S0,
+                                    S1);
 }
 
 // 64x64 tile for grids that would otherwise leave CUs idle or need a
@@ -958,11 +980,13 @@ inline bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 
 // two wave groups (branch-free shapes whose K slices are whole K tiles only);
 // 3 = 128x256 (four waves), 4 = 128x128 (eight waves) direct-to-LDS, for
 // branch-free shapes only (otherwise the staged shape of the same size runs).
-constexpr int kTileShapes = 7;
-constexpr int kTileM[kTileShapes] = {128, 128, 64, 128, 128, 64, 64};
-constexpr int kTileN[kTileShapes] = {256, 128, 128, 256, 128, 64, 64};
-constexpr int kStagedFallback[kTileShapes] = {0, 1, 2, 0, 1, 2, 2};
-constexpr int kTileK[kTileShapes] = {16, 16, 16, 16, 16, 32, 64};  // K granule of a slice
+// 7 = 64x128 (four waves) direct-to-LDS.
+constexpr int kTileShapes = 8;
+constexpr int kVariantTiles = 7;  // those a caller may choose (sgemm_device_variant)
+constexpr int kTileM[kTileShapes] = {128, 128, 64, 128, 128, 64, 64, 64};
+constexpr int kTileN[kTileShapes] = {256, 128, 128, 256, 128, 64, 64, 128};
+constexpr int kStagedFallback[kTileShapes] = {0, 1, 2, 0, 1, 2, 2, 2};
+constexpr int kTileK[kTileShapes] = {16, 16, 16, 16, 16, 32, 64, 16};  // K granule of a slice
 
 struct SgemmPlan {
   int tile;    // index into kTileM / kTileN
@@ -996,8 +1020,8 @@ bool buffer_path(bool aligned, int lda, long long sa, int ldb, long long sb, uin
   // B chunks past column n lie in B's padding or next row and only feed
   // output columns that are never stored, so n itself may be ragged.
   const bool vec = (k % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) && (sb % 4 == 0) && aligned;
-  const bool k_ok = tile >= 5 ? true : (k % kBK == 0) && (k_len % kBK == 0);
-  return vec && k_ok && (size_t)(m + 128) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
+  const bool k_ok = tile == 5 || tile == 6 ? true : (k % kBK == 0) && (k_len % kBK == 0);
+  return vec && k_ok && (size_t)(m + 192) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
 }
 
 // Plan choice: the (tile shape, K slices) pair with the least estimated time.
@@ -1012,7 +1036,7 @@ bool buffer_path(bool aligned, int lda, long long sa, int ldb, long long sb, uin
 // shapes, the C4 and Z-Image block products, their 32-row tails, tall and
 // wide panels); the chosen plan is within 1 % of the measured best on
 // average and within 5 % at all but one shape.
-constexpr int kTileOcc[kTileShapes] = {2, 3, 4, 3, 5, 4, 2};
+constexpr int kTileOcc[kTileShapes] = {2, 3, 4, 3, 5, 4, 2, 5};
 constexpr double kTileEffW[kTileShapes][5] = {
     {0.776, 0.883},                       // 128x256 staged
     {0.726, 0.837, 0.913},                // 128x128 staged
@@ -1020,7 +1044,8 @@ constexpr double kTileEffW[kTileShapes][5] = {
     {0.900, 0.975, 0.948},                // 128x256 direct
     {0.935, 0.971, 0.976, 0.967, 0.967},  // 128x128 direct, eight waves
     {0.606, 0.766, 0.846, 0.931},         // 64x64 direct, K tile 32
-    {0.772, 0.911}};                      // 64x64 direct, K tile 64
+    {0.772, 0.911},                       // 64x64 direct, K tile 64
+    {0.730, 0.850, 0.900, 0.930, 0.945}}; // 64x128 direct
 
 // scalar_loads: the register-staged kernels read the operands with predicated
 // 32-bit loads (k or n not a multiple of 4, unaligned rows), about 1.5x slower
@@ -1054,7 +1079,7 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
   // The eight-wave 128x128 kernel is tried first and is only replaced by a
   // plan more than 1 % cheaper (near ties keep the established kernel; the
   // model is accurate to a few per cent).
-  static const int kTileOrder[kTileShapes] = {4, 3, 0, 1, 2, 5, 6};
+  static const int kTileOrder[kTileShapes] = {4, 3, 0, 1, 2, 5, 6, 7};
   const bool scalar = !((k % 4 == 0) && (n % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) &&
                         (sb % 4 == 0) && aligned);
   SgemmPlan best = make_plan(0, 1, k);
@@ -1159,6 +1184,10 @@ hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long
       hipLaunchKernelGGL(sgemm_f32_dl128w8_kernel, grid, dim3(512), 0, stream, a, b, out, (int)m, (int)n, (int)k,
                          tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
+    case 7:
+      hipLaunchKernelGGL(sgemm_f32_dl64x128_kernel, grid, dim3(256), 0, stream, a, b, out, (int)m, (int)n, (int)k,
+                         tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
+      break;
     case 0:
       launch_tile<128, 256>(buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda, ldb,
                             ldo, res, ldr, p.k_len, sa, sb, sc);
@@ -1259,7 +1288,7 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
     // slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger one faster
     // (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
     const bool small = (uint64_t)n * k < (1u << 20);
-    const double bias = small ? (rows.splits > 1 ? 1.2 : 0.0) : -0.06 * s.cost_us;
+    const double bias = small ? (rows.splits > 1 ? 1.6 : 0.0) : -0.06 * s.cost_us;
     if (rows.us + bias < s.cost_us) {
       s = SgemmSchedule{};
       s.few_rows = true;
@@ -1431,6 +1460,29 @@ int launch_sgemm_f32_noalloc(const float* a, const float* b, float* c, uint32_t 
              : PROM_DETAIL_HIP_LAUNCH_FAILED;
 }
 
+namespace {
+
+template <int kBM>
+void launch_geglu_tiles(const float* a, int lda, const float* w, float* h, int ldh, uint32_t m, uint32_t f, uint32_t k,
+                        hipStream_t stream) {
+  const int tiles_m = (int)((m + kBM - 1) / kBM), tiles_n = (int)(f / 64);
+  hipLaunchKernelGGL(sgemm_f32_dl128h_geglu_kernel<kBM>, dim3((unsigned)(tiles_m * tiles_n)), dim3(4 * kBM), 0, stream,
+                     a, w, h, (int)m, (int)f, (int)k, tiles_m, tiles_n, lda, (int)(2 * f), ldh);
+}
+
+// Rows per tile of the GeGLU product: the height with the least padded work, a
+// taller tile on ties.  At 2048 x 2 * 16384, us for 64 / 128 / 192 rows per tile: 64
+// tokens 90 / 127 / 184, 130 tokens 192 / 239 / 184, 192 tokens 205 / 240 / 199,
+// 256 tokens 258 / 248 / 359, 300 tokens 324 / 357 / 357, 512 tokens 519 / 503 / 532.
+// The 64-row tile runs 4 % below the 128-row one; 192 pays as the only tile row.
+int geglu_height(uint32_t m) {
+  const double r64 = (double)((m + 63) / 64) * 64 * 1.04, r128 = (double)((m + 127) / 128) * 128;
+  if (m > 128 && m <= 192) return 192;
+  return r64 < r128 ? 64 : 128;
+}
+
+}  // namespace
+
 hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float* h, int ldh, uint32_t m, uint32_t f,
                                   uint32_t k, hipStream_t stream) {
   if (m == 0 || f == 0 || k == 0) return hipErrorNotSupported;
@@ -1445,15 +1497,17 @@ hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float
   const bool ok = f % 64 == 0 && buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k, (int)k, 4) &&
                   ldh % 4 == 0 && aligned16(h);
   if (!ok) return hipErrorNotSupported;
-  const int tiles_m = (int)((m + 127) / 128), tiles_n = (int)(f / 64);
-  hipLaunchKernelGGL(sgemm_f32_dl128w8_geglu_kernel, dim3((unsigned)(tiles_m * tiles_n)), dim3(512), 0, stream, a, w,
-                     h, (int)m, (int)f, (int)k, tiles_m, tiles_n, lda, ldb, ldh);
+  switch (geglu_height(m)) {
+    case 64: launch_geglu_tiles<64>(a, lda, w, h, ldh, m, f, k, stream); break;
+    case 192: launch_geglu_tiles<192>(a, lda, w, h, ldh, m, f, k, stream); break;
+    default: launch_geglu_tiles<128>(a, lda, w, h, ldh, m, f, k, stream); break;
+  }
   return hipGetLastError();
 }
 
 hipError_t launch_sgemm_f32_variant(const float* a, const float* b, float* c, uint32_t m, uint32_t n, uint32_t k,
                                     uint32_t tile, uint32_t k_slices, hipStream_t stream) {
-  if (tile >= (uint32_t)kTileShapes || k_slices < 1u || k_slices > 16u) return hipErrorInvalidValue;
+  if (tile >= (uint32_t)kVariantTiles || k_slices < 1u || k_slices > 16u) return hipErrorInvalidValue;
   const SgemmPlan p = make_plan((int)tile, (int)k_slices, k);
   const bool aligned = aligned16(a) && aligned16(b);
   if (p.splits != (int)k_slices || (tile >= 3 && !buffer_path(aligned, (int)k, 0, (int)n, 0, m, n, k, p.k_len, tile)))
