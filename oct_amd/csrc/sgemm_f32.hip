@@ -118,14 +118,15 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
 
   float ra[T::kAPer];
   float rb[4 * T::kBVec];
-  // Branch-free loads (kBuf: K of this slice is a multiple of the K tile): buffer
-  // loads return zero for rows of A at or past M and past the end of B; columns of
-  // B at or past N only feed output columns that are never stored.
+  // kBuf: 16-byte buffer loads at any 4-byte alignment, without branches: they return
+  // zero for rows of A at or past M and rows of B at or past K; columns of B at or
+  // past N only feed output columns that are never stored.  A's values past K (another
+  // row's) are cleared in the last K tile.
+  // The ranges end with the last value of the last row.
   const __amdgpu_buffer_rsrc_t rsa = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)A, (short)0, kBuf ? (int)(((size_t)M * lda - (gridDim.y > 1 ? (size_t)blockIdx.y * k_len : 0)) * 4) : 0,
-      0x00020000);
-  const __amdgpu_buffer_rsrc_t rsb =
-      __builtin_amdgcn_make_buffer_rsrc((void*)B, (short)0, kBuf ? (int)((size_t)K * ldb * 4) : 0, 0x00020000);
+      (void*)A, (short)0, kBuf ? (int)(((size_t)(M - 1) * lda + K) * 4) : 0, 0x00020000);
+  const __amdgpu_buffer_rsrc_t rsb = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)B, (short)0, kBuf ? (int)(((size_t)(K - 1) * ldb + N) * 4) : 0, 0x00020000);
 
   auto load_tile = [&](int k0) {
     const int gr = row0 + a_row;
@@ -134,18 +135,23 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
 #pragma unroll
       for (int h = 0; h < T::kAPer / 4; ++h) {
         const int gk = k0 + a_k + 4 * h;
-        const floatx4 v =
-            __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsa, (uint32_t)((gr * lda + gk) * 4), 0, 0));
+        const floatx4 v = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsa, (uint32_t)((gr * lda + gk) * 4), 0, 0));
         ra[4 * h + 0] = v.x;
         ra[4 * h + 1] = v.y;
         ra[4 * h + 2] = v.z;
         ra[4 * h + 3] = v.w;
       }
+      if (k0 + kBK > K) {
+#pragma unroll
+        for (int j = 0; j < T::kAPer; ++j)
+          if (k0 + a_k + j >= K) ra[j] = 0.f;
+      }
 #pragma unroll
       for (int h = 0; h < T::kBVec; ++h) {
         const int gk = k0 + b_k + T::kBRowStep * h;
-        const floatx4 v =
-            __builtin_bit_cast(floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsb, (uint32_t)((gk * ldb + gn) * 4), 0, 0));
+        const floatx4 v = __builtin_bit_cast(
+            floatx4, __builtin_amdgcn_raw_buffer_load_b128(rsb, (uint32_t)((gk * ldb + gn) * 4), 0, 0));
         rb[4 * h + 0] = v.x;
         rb[4 * h + 1] = v.y;
         rb[4 * h + 2] = v.z;
@@ -268,8 +274,8 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
     for (int j = 0; j < T::kNI; ++j) store_block(acc[i][j], i, j);
 }
 
-// Direct-to-LDS variant for the branch-free shapes (k, n, lda, ldb multiples
-// of 4, every slice a multiple of the K tile): A and B tiles go from HBM to LDS
+// Direct-to-LDS variant for operands with 16-byte rows (k, lda, ldb multiples of
+// 4): A and B tiles go from HBM to LDS
 // with buffer_load ... lds (16 bytes per lane, no register staging), which
 // frees the staging registers for a third workgroup per CU (128x256) and
 // removes the transposing LDS stores.
@@ -299,7 +305,14 @@ struct DlCfg {
 // are a gate block and its up block (tile columns 0-31 gate, 32-63 up, 64-95
 // gate + 32, 96-127 up + 32); the epilogue stores gelu_tanh(gate) * up, N
 // columns in all.
-template <int kBN, int kBM, bool kGeGLU = false>
+//
+// kTail (128x128 tiles, K a multiple of 4 but not of the K tile): the last tile's B
+// rows past K read zero (outside the buffer range), and its A columns past K, which
+// the transfers fill from the next row, are cleared in LDS before that tile is used.
+// The sums are taken in two, of the first and the second half of each K tile: the
+// 64x64 tiles, the other kernels for such a K, add two as well, and 4097x3001x513 keeps their error (2.9e-7 of the
+// result against 64 bits; 4.1e-7 in one chain) at 128x128's speed: 114 us, 124 before.
+template <int kBN, int kBM, bool kGeGLU = false, bool kTail = false>
 __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, const float* __restrict__ B, float* C,
                                                   int M, int N, int K, int tiles_m, int tiles_n, int lda, int ldb,
                                                   int ldc, const float* R, int ldr, int k_len, long long sa,
@@ -406,10 +419,14 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
   }
 
   floatx16 acc[kMI][kNI];
+  floatx16 acc_odd[kTail ? kMI : 1][kTail ? kNI : 1];  // kTail: the second half of each K tile
 #pragma unroll
   for (int i = 0; i < kMI; ++i)
 #pragma unroll
-    for (int j = 0; j < kNI; ++j) acc[i][j] = floatx16{};
+    for (int j = 0; j < kNI; ++j) {
+      acc[i][j] = floatx16{};
+      if constexpr (kTail) acc_odd[i][j] = floatx16{};
+    }
 
   auto compute = [&](const char* st) {
 #pragma unroll
@@ -432,15 +449,28 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
 #pragma unroll
         for (int mi = 0; mi < kMI; ++mi)
 #pragma unroll
-          for (int ni = 0; ni < kNI; ++ni)
-            acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mi][j], b[ni], acc[mi][ni], 0, 0, 0);
+          for (int ni = 0; ni < kNI; ++ni) {
+            floatx16& sum = kTail && p == 1 ? acc_odd[kTail ? mi : 0][kTail ? ni : 0] : acc[mi][ni];
+            sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mi][j], b[ni], sum, 0, 0, 0);
+          }
       }
       // Keep each half's operand reads within the half: bounds register pressure.
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
-  const int k_tiles = K / kBK;
+  const int k_tiles = kTail ? (K + kBK - 1) / kBK : K / kBK;
+  auto settle_last = [&](char* st) {
+    const int c0 = (K % kBK) / 4;
+    if (c0 == 0) return;  // a slice of whole tiles
+    const int nc = kBK / 4 - c0;
+    for (int e = tid; e < kBM * nc; e += 64 * kWaves) {
+      const int r = e / nc;
+      const int c = c0 + e % nc;
+      *reinterpret_cast<floatx4*>(st + r * 64 + ((c ^ ((r >> 2) & 3)) << 4)) = floatx4{};
+    }
+    __syncthreads();
+  };
   issue(S0, 0);
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
@@ -452,12 +482,24 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
     compute(S0);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    if (kt + 2 < k_tiles) issue(S0, (kt + 2) * kBK);
+    if (kt + 2 < k_tiles)
+      issue(S0, (kt + 2) * kBK);
+    else if constexpr (kTail)
+      settle_last(S1);
     compute(S1);
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
   }
-  if (kt < k_tiles) compute(S0);  // odd count: the last tile was issued into S0
+  if (kt < k_tiles) {  // odd count: the last tile was issued into S0
+    if constexpr (kTail) settle_last(S0);
+    compute(S0);
+  }
+  if constexpr (kTail) {
+#pragma unroll
+    for (int i = 0; i < kMI; ++i)
+#pragma unroll
+      for (int j = 0; j < kNI; ++j) acc[i][j] += acc_odd[i][j];
+  }
 
   if constexpr (kGeGLU) {
     // acc[0][0]: gate columns col0 + 32 wn + lrow, acc[0][1]: the same up columns
@@ -513,6 +555,7 @@ __global__ __launch_bounds__(256, 3) void sgemm_f32_dl256_kernel(const float* __
 // row offsets among them, allow seven waves per SIMD).  Two or four
 // workgroups per CU measured the same at 4096^3 (921 us), four 4 % slower
 // at 8192 x 8192 x 2048.
+template <bool kTail>
 __global__ __launch_bounds__(512, 1) void sgemm_f32_dl128w8_kernel(const float* __restrict__ A,
                                                                    const float* __restrict__ B, float* C, int M,
                                                                    int N, int K, int tiles_m, int tiles_n, int lda,
@@ -521,7 +564,8 @@ __global__ __launch_bounds__(512, 1) void sgemm_f32_dl128w8_kernel(const float* 
                                                                    long long sc) {
   __shared__ __attribute__((aligned(1024))) char S0[DlCfg<128>::kStage];
   __shared__ __attribute__((aligned(1024))) char S1[DlCfg<128>::kStage];
-  sgemm_f32_dl_body<128, 128>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa, sb, sc, S0, S1);
+  sgemm_f32_dl_body<128, 128, false, kTail>(A, B, C, M, N, K, tiles_m, tiles_n, lda, ldb, ldc, R, ldr, k_len, sa,
+                                              sb, sc, S0, S1);
 }
 
 // The same with 64 rows (four waves of 32x64), for row counts that 128 divides
@@ -921,55 +965,50 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
   if (lane == 0) y[row] = acc;
 }
 
-// C = sum over `splits` slabs of P (fixed order: deterministic) + R.
+// C = sum over `splits` (at most 16) slabs of P (fixed order: deterministic) + R, 4
+// columns per thread, one workgroup row-slice per (blockIdx.x, row): no per-element
+// 64-bit division, and 16-byte loads at any 4-byte alignment, all issued before the
+// adds.  The last n % 4 columns are taken one by one.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float* __restrict__ P, float* C, int M, int N,
                                                             int ldc, int splits, const float* R, int ldr) {
-  const size_t total = (size_t)M * N;
+  typedef float floatx4u __attribute__((ext_vector_type(4), aligned(4)));
+  const int c = 4 * (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  if (c >= N) return;
   const size_t slab = (size_t)M * N;
-  for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += (size_t)gridDim.x * blockDim.x) {
-    const size_t row = idx / N;
-    const size_t col = idx - row * N;
-    float v = P[idx];
-    for (int s = 1; s < splits; ++s) v += P[(size_t)s * slab + idx];
-    if (R != nullptr) v += R[row * ldr + col];
-    C[row * ldc + col] = v;
-  }
-}
-
-// Same sum, 4 columns per thread (N, ldc, ldr multiples of 4, 16-byte aligned
-// C and R): one workgroup row-slice per (blockIdx.x, row), no per-element
-// 64-bit division; the slabs are read with 128-bit loads, all issued before
-// the adds (same order of additions as the scalar kernel).
-__global__ __launch_bounds__(256) void splitk_reduce4_kernel(const float* __restrict__ P, float* C, int M, int N,
-                                                             int ldc, int splits, const float* R, int ldr) {
-  const int n4 = N >> 2;
-  const int c4 = (int)(blockIdx.x * blockDim.x + threadIdx.x);
-  if (c4 >= n4) return;
-  const size_t slab4 = (size_t)M * n4;
-  const floatx4* P4 = reinterpret_cast<const floatx4*>(P);
   for (int row = (int)blockIdx.y; row < M; row += (int)gridDim.y) {
-    const size_t i = (size_t)row * n4 + c4;
-    floatx4 part[16];
+    const float* p = P + (size_t)row * N + c;
+    float* out = C + (size_t)row * ldc + c;
+    const float* res = R != nullptr ? R + (size_t)row * ldr + c : nullptr;
+    if (c + 4 <= N) {
+      floatx4 part[16];
 #pragma unroll
-    for (int s = 0; s < 16; ++s)
-      if (s < splits) part[s] = P4[(size_t)s * slab4 + i];
-    floatx4 v = part[0];
+      for (int s = 0; s < 16; ++s)
+        if (s < splits) part[s] = *reinterpret_cast<const floatx4u*>(p + (size_t)s * slab);
+      floatx4 v = part[0];
 #pragma unroll
-    for (int s = 1; s < 16; ++s)
-      if (s < splits) {
-        v.x += part[s].x;
-        v.y += part[s].y;
-        v.z += part[s].z;
-        v.w += part[s].w;
+      for (int s = 1; s < 16; ++s)
+        if (s < splits) {
+          v.x += part[s].x;
+          v.y += part[s].y;
+          v.z += part[s].z;
+          v.w += part[s].w;
+        }
+      if (res != nullptr) {
+        const floatx4 r = *reinterpret_cast<const floatx4u*>(res);
+        v.x += r.x;
+        v.y += r.y;
+        v.z += r.z;
+        v.w += r.w;
       }
-    if (R != nullptr) {
-      const floatx4 r = reinterpret_cast<const floatx4*>(R + (size_t)row * ldr)[c4];
-      v.x += r.x;
-      v.y += r.y;
-      v.z += r.z;
-      v.w += r.w;
+      *reinterpret_cast<floatx4u*>(out) = v;
+    } else {
+      for (int j = 0; j < N - c; ++j) {
+        float v = p[j];
+        for (int s = 1; s < splits; ++s) v += p[(size_t)s * slab + j];
+        if (res != nullptr) v += res[j];
+        out[j] = v;
+      }
     }
-    reinterpret_cast<floatx4*>(C + (size_t)row * ldc)[c4] = v;
   }
 }
 
@@ -1009,19 +1048,22 @@ SgemmPlan make_plan(int tile, int splits, uint32_t k) {
   return p;
 }
 
-// True when the buffer-load kernels apply: 128-bit aligned operands, every
-// slice length a multiple of the K tile and every 32-bit byte offset (rows up
-// to M + 128, all of B plus a tile row) in range.
-// `aligned`: both operand base addresses are 16-byte aligned.  The 128-wide
-// direct kernels need every slice to be whole K tiles of 16; the 64x64 ones
-// (tiles 5 and 6) take a K tail (k % 4 == 0) in the last tile of each product.
-bool buffer_path(bool aligned, int lda, long long sa, int ldb, long long sb, uint32_t m, uint32_t n, uint32_t k,
-                 int k_len, int tile = 4) {
+// True when the direct-to-LDS kernels apply: operands of 16-byte aligned rows and
+// every 32-bit byte offset (rows up to M + 192, all of B plus a tile row) in range.
+// `aligned`: both operand base addresses are 16-byte aligned.  A K tail (k % 4 == 0)
+// is taken in the last tile of the last slice (by tiles 4, 5 and 6).
+bool buffer_path(bool aligned, int lda, long long sa, int ldb, long long sb, uint32_t m, uint32_t n, uint32_t k) {
   // B chunks past column n lie in B's padding or next row and only feed
   // output columns that are never stored, so n itself may be ragged.
   const bool vec = (k % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) && (sb % 4 == 0) && aligned;
-  const bool k_ok = tile == 5 || tile == 6 ? true : (k % kBK == 0) && (k_len % kBK == 0);
-  return vec && k_ok && (size_t)(m + 192) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
+  return vec && (size_t)(m + 192) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
+}
+
+// True when the register-staged kernels read through buffer descriptors: every 32-bit
+// byte offset (rows up to M + 128, B to a K tile past its end) in range, whatever the
+// alignment.
+bool staged_buffer_path(int lda, int ldb, uint32_t m, uint32_t n, uint32_t k) {
+  return (size_t)(m + 128) * lda * 4 < (1ull << 31) && (((size_t)k + 16) * ldb + n + 256) * 4 < (1ull << 31);
 }
 
 // Plan choice: the (tile shape, K slices) pair with the least estimated time.
@@ -1047,10 +1089,21 @@ constexpr double kTileEffW[kTileShapes][5] = {
     {0.772, 0.911},                       // 64x64 direct, K tile 64
     {0.780, 0.870, 0.920, 0.945, 0.960}}; // 64x128 direct
 
-// scalar_loads: the register-staged kernels read the operands with predicated
-// 32-bit loads (k or n not a multiple of 4, unaligned rows), about 1.5x slower
-// per K step than with 128-bit loads (measured at 4097x3001x513).
-double plan_cost(const SgemmPlan& p, uint32_t m, uint32_t n, uint32_t batch, bool scalar_loads = false) {
+// How the register-staged kernels read operands whose rows are not 16-byte aligned:
+// through buffer descriptors (16-byte loads at any alignment: 1 to 13 % slower than
+// estimated in the median of 46 ragged shapes, the slowest tenth 20 to 30 %; counted
+// as 15 % and 1.3 us, so that near ties keep the padded copies: 3261x340x4070 100 us against 134
+// on copies, 3877x2818x70 29 against 33) or, past the descriptors' 2 GiB, with
+// predicated 32-bit loads (about 1.5x slower per K step).
+enum class Rows { kAligned, kUnaligned, kScalar };
+
+Rows operand_rows(bool aligned, int lda, long long sa, int ldb, long long sb, uint32_t m, uint32_t n, uint32_t k) {
+  if (k % 4 == 0 && n % 4 == 0 && lda % 4 == 0 && ldb % 4 == 0 && sa % 4 == 0 && sb % 4 == 0 && aligned)
+    return Rows::kAligned;
+  return staged_buffer_path(lda, ldb, m, n, k) ? Rows::kUnaligned : Rows::kScalar;
+}
+
+double plan_cost(const SgemmPlan& p, uint32_t m, uint32_t n, uint32_t batch, Rows rows = Rows::kAligned) {
   const int t = p.tile;
   const double w_total = (double)((m + kTileM[t] - 1) / kTileM[t]) * ((n + kTileN[t] - 1) / kTileN[t]) * p.splits *
                          batch;
@@ -1065,7 +1118,8 @@ double plan_cost(const SgemmPlan& p, uint32_t m, uint32_t n, uint32_t batch, boo
     const int w = (int)std::ceil(rest / 256.0);
     us += w * k_tiles * t16 / eff(w);
   }
-  if (scalar_loads && t < 3) us *= 1.5;
+  if (t < 3 && rows == Rows::kUnaligned) us = 1.15 * us + 1.3;
+  if (t < 3 && rows == Rows::kScalar) us *= 1.5;
   us += 3.45 + 1.72 * (full + (rest > 0 ? 1.0 : 0.0));
   if (p.splits > 1) us += 1.46 + (double)(p.splits + 1) * m * n * 4.0 / 3.5e6;
   return us;
@@ -1080,8 +1134,7 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
   // plan more than 1 % cheaper (near ties keep the established kernel; the
   // model is accurate to a few per cent).
   static const int kTileOrder[kTileShapes] = {4, 3, 0, 1, 2, 5, 6, 7};
-  const bool scalar = !((k % 4 == 0) && (n % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) &&
-                        (sb % 4 == 0) && aligned);
+  const Rows kind = operand_rows(aligned, lda, sa, ldb, sb, m, n, k);
   SgemmPlan best = make_plan(0, 1, k);
   double best_cost = 1e300;
   for (int t : kTileOrder) {
@@ -1091,8 +1144,11 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
       const SgemmPlan p = make_plan(t, s, k);
       if (p.splits != s) continue;
       if (p.splits > 1 && (uint64_t)p.splits * m * n > max_partial_floats) continue;
-      if (t >= 3 && !buffer_path(aligned, lda, sa, ldb, sb, m, n, k, p.k_len, t)) continue;
-      const double c = plan_cost(p, m, n, batch, scalar);
+      if (t >= 3 && !buffer_path(aligned, lda, sa, ldb, sb, m, n, k)) continue;
+      // K tails: the 64x64 tiles, and 128x128, whose offsets (to a K tile past B) stay
+      // below 2^32 if B has a K tile itself
+      if ((t == 3 || t == 7 || (t == 4 && k < (uint32_t)kBK)) && k % kBK != 0) continue;
+      const double c = plan_cost(p, m, n, batch, kind);
       if (c < best_cost * 0.99) {
         best_cost = c;
         best = p;
@@ -1120,19 +1176,10 @@ void launch_tile(bool buf, bool vec, dim3 grid, hipStream_t stream, const float*
 // c = the sum of `splits` slices of partial (m * n floats apart) + residual.
 hipError_t launch_splitk_reduce(const float* partial, float* c, uint32_t m, uint32_t n, int ldc, int splits,
                                 const float* residual, int ldr, hipStream_t stream) {
-  const bool vec4 = n % 4 == 0 && ldc % 4 == 0 && aligned16(c) &&
-                    (residual == nullptr || (ldr % 4 == 0 && aligned16(residual)));
-  if (vec4 && splits <= 16) {
-    const unsigned bx = (unsigned)((n / 4 + 255) / 256);
-    const unsigned by = (unsigned)std::min<uint32_t>(m, std::max(1u, 8192u / bx));
-    hipLaunchKernelGGL(splitk_reduce4_kernel, dim3(bx, by), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
-                       splits, residual, ldr);
-  } else {
-    const size_t total = (size_t)m * n;
-    const unsigned blocks = (unsigned)std::min((size_t)8192, (total + 255) / 256);
-    hipLaunchKernelGGL(splitk_reduce_kernel, dim3(blocks), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc,
-                       splits, residual, ldr);
-  }
+  const unsigned bx = (unsigned)(((size_t)n + 1023) / 1024);
+  const unsigned by = (unsigned)std::min<uint32_t>(m, std::max(1u, 8192u / bx));
+  hipLaunchKernelGGL(splitk_reduce_kernel, dim3(bx, by), dim3(256), 0, stream, partial, c, (int)m, (int)n, ldc, splits,
+                     residual, ldr);
   return hipGetLastError();
 }
 
@@ -1145,8 +1192,9 @@ hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long
   const bool split = p.splits > 1;
   const bool vec = (k % 4 == 0) && (n % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) &&
                    (sb % 4 == 0) && aligned16(a) && aligned16(b);
-  const bool buf = buffer_path(aligned16(a) && aligned16(b), lda, sa, ldb, sb, m, n, k, p.k_len, p.tile);
+  const bool buf = buffer_path(aligned16(a) && aligned16(b), lda, sa, ldb, sb, m, n, k);
   const int tile = (p.tile >= 3 && !buf) ? kStagedFallback[p.tile] : p.tile;
+  const bool staged_buf = staged_buffer_path(lda, ldb, m, n, k);
   const int bm = kTileM[tile], bn = kTileN[tile];
   const int tiles_m = (int)((m + bm - 1) / bm);
   const int tiles_n = (int)((n + bn - 1) / bn);
@@ -1182,24 +1230,28 @@ hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long
                          tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
     case 4:
-      hipLaunchKernelGGL(sgemm_f32_dl128w8_kernel, grid, dim3(512), 0, stream, a, b, out, (int)m, (int)n, (int)k,
-                         tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
+      if (k % kBK != 0)
+        hipLaunchKernelGGL(sgemm_f32_dl128w8_kernel<true>, grid, dim3(512), 0, stream, a, b, out, (int)m,
+                           (int)n, (int)k, tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
+      else
+        hipLaunchKernelGGL(sgemm_f32_dl128w8_kernel<false>, grid, dim3(512), 0, stream, a, b, out, (int)m,
+                           (int)n, (int)k, tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
     case 7:
       hipLaunchKernelGGL(sgemm_f32_dl64x128_kernel, grid, dim3(256), 0, stream, a, b, out, (int)m, (int)n, (int)k,
                          tiles_m, tiles_n, lda, ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
     case 0:
-      launch_tile<128, 256>(buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda, ldb,
-                            ldo, res, ldr, p.k_len, sa, sb, sc);
+      launch_tile<128, 256>(staged_buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda,
+                          ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
     case 1:
-      launch_tile<128, 128>(buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda, ldb,
-                            ldo, res, ldr, p.k_len, sa, sb, sc);
+      launch_tile<128, 128>(staged_buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda,
+                          ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
     default:
-      launch_tile<64, 128>(buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda, ldb,
-                           ldo, res, ldr, p.k_len, sa, sb, sc);
+      launch_tile<64, 128>(staged_buf, vec, grid, stream, a, b, out, (int)m, (int)n, (int)k, tiles_m, tiles_n, lda,
+                         ldb, ldo, res, ldr, p.k_len, sa, sb, sc);
       break;
   }
   const hipError_t e = hipGetLastError();
@@ -1214,8 +1266,9 @@ hipError_t run_sgemm_plan(const SgemmPlan& p, const float* a, int lda, long long
 struct SgemmSchedule {
   bool gemv;
   bool few_rows;
-  SgemmRowsPlan rows;  // few_rows
+  SgemmRowsPlan rows;  // few_rows, tail_rows
   bool tail_split;
+  bool tail_rows;      // the second product runs on the few-rows kernel
   bool repack;         // A, B copied first to [m][k4] and [k4][n4], 16-byte rows, zero padding
   uint32_t k4, n4;     // padded K and B row stride when repacking
   uint32_t head_rows;  // rows of the first product (m without a tail split)
@@ -1223,18 +1276,31 @@ struct SgemmSchedule {
   double cost_us;      // plan-model estimate of the queued work
 };
 
+// Whether the few-rows kernel takes an m x n x k product that the tiles are estimated
+// to run in tiles_us.  The two models meet where both are off: a sliced product of a
+// small B measured slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger
+// one faster (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
+bool few_rows_win(uint32_t m, uint32_t n, uint32_t k, int lda, int ldb, double tiles_us, uint64_t max_partial_floats,
+                  SgemmRowsPlan* rows) {
+  if (!sgemm_rows_take(m, k, lda, ldb, 1)) return false;
+  *rows = plan_sgemm_rows(m, n, k, false, max_partial_floats);
+  const bool small = (uint64_t)n * k < (1u << 20);
+  const double bias = small ? (rows->splits > 1 ? 1.6 : 0.0) : -0.06 * tiles_us;
+  return rows->us + bias < tiles_us;
+}
+
 // One or two products (tail split) of an m x n x k problem with the given
 // operand description.
 SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint32_t n, uint32_t k,
                                 uint64_t max_partial_floats) {
   SgemmSchedule s{};
   s.head_rows = m;
-  const bool scalar = !((k % 4 == 0) && (n % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && aligned);
+  const Rows kind = operand_rows(aligned, lda, 0, ldb, 0, m, n, k);
   s.plan[0] = plan_sgemm(aligned, lda, 0, ldb, 0, m, n, k, 1, max_partial_floats);
-  s.cost_us = plan_cost(s.plan[0], m, n, 1, scalar);
+  s.cost_us = plan_cost(s.plan[0], m, n, 1, kind);
   // A partial last row of 128-row tiles runs nearly empty for the whole K depth
   // (M = 1056: a 32-row tail in 9 tile rows).  When the estimate favours it, the
-  // rows past the last full tile row run as a second product (usually K-split)
+  // rows past the last full tile row run as a second product (K-split or few-rows)
   // after the rest, on the same stream.  The tail starts 128 rows in, so its A
   // keeps the alignment of a when lda is a multiple of 4.
   const uint32_t tail = m % 128u;
@@ -1243,9 +1309,17 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
     const bool tail_aligned = aligned && (lda % 4 == 0);
     const SgemmPlan ph = plan_sgemm(aligned, lda, 0, ldb, 0, head, n, k, 1, max_partial_floats);
     const SgemmPlan pt = plan_sgemm(tail_aligned, lda, 0, ldb, 0, tail, n, k, 1, max_partial_floats);
-    const double split_cost = plan_cost(ph, head, n, 1, scalar) + plan_cost(pt, tail, n, 1, scalar);
+    double tail_us = plan_cost(pt, tail, n, 1, kind);
+    // The few-rows kernel takes short K's tails, which the tiles cannot slice (one row
+    // of 3001x516: 5.5 us against 10); a long K's are 1 or 2 % of the whole either way.
+    SgemmRowsPlan rows;
+    const bool tail_rows = k < 1024u && few_rows_win(tail, n, k, lda, ldb, tail_us, max_partial_floats, &rows);
+    if (tail_rows) tail_us = rows.us;
+    const double split_cost = plan_cost(ph, head, n, 1, kind) + tail_us;
     if (split_cost < s.cost_us) {
       s.tail_split = true;
+      s.tail_rows = tail_rows;
+      if (tail_rows) s.rows = rows;
       s.head_rows = head;
       s.plan[0] = ph;
       s.plan[1] = pt;
@@ -1283,20 +1357,13 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
       }
     }
   }
-  if (sgemm_rows_take(m, k, lda, ldb, 1)) {
-    const SgemmRowsPlan rows = plan_sgemm_rows(m, n, k, false, max_partial_floats);
-    // The two models meet where both are off: a sliced product of a small B measured
-    // slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger one faster
-    // (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
-    const bool small = (uint64_t)n * k < (1u << 20);
-    const double bias = small ? (rows.splits > 1 ? 1.6 : 0.0) : -0.06 * s.cost_us;
-    if (rows.us + bias < s.cost_us) {
-      s = SgemmSchedule{};
-      s.few_rows = true;
-      s.rows = rows;
-      s.head_rows = m;
-      s.cost_us = rows.us;
-    }
+  SgemmRowsPlan rows;
+  if (few_rows_win(m, n, k, lda, ldb, s.cost_us, max_partial_floats, &rows)) {
+    s = SgemmSchedule{};
+    s.few_rows = true;
+    s.rows = rows;
+    s.head_rows = m;
+    s.cost_us = rows.us;
   }
   return s;
 }
@@ -1315,18 +1382,20 @@ hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, c
     hipLaunchKernelGGL(gemv_f32_kernel, dim3((m + 3) / 4), dim3(256), 0, stream, a, b, c, (int)m, (int)k);
     return hipGetLastError();
   }
-  if (s.few_rows) {
+  auto run_rows = [&](const float* ap, float* cp, const float* rp, uint32_t rows) {
     SgemmRowsPlan p = s.rows;
     float* part = nullptr;
     if (p.splits > 1) {
-      part = partial != nullptr ? partial : static_cast<float*>(staging(6, (size_t)p.splits * m * n * sizeof(float)));
+      part = partial != nullptr ? partial
+                                : static_cast<float*>(staging(6, (size_t)p.splits * rows * n * sizeof(float)));
       if (part == nullptr) p.splits = 1;
     }
-    if (p.splits == 1) return launch_sgemm_rows(p, a, lda, b, ldb, c, ldc, m, n, k, residual, ldr, stream);
-    const hipError_t e = launch_sgemm_rows(p, a, lda, b, ldb, part, (int)n, m, n, k, nullptr, 0, stream);
+    if (p.splits == 1) return launch_sgemm_rows(p, ap, lda, b, ldb, cp, ldc, rows, n, k, rp, ldr, stream);
+    const hipError_t e = launch_sgemm_rows(p, ap, lda, b, ldb, part, (int)n, rows, n, k, nullptr, 0, stream);
     if (e != hipSuccess || !reduce) return e;
-    return launch_splitk_reduce(part, c, m, n, ldc, p.splits, residual, ldr, stream);
-  }
+    return launch_splitk_reduce(part, cp, rows, n, ldc, p.splits, rp, ldr, stream);
+  };
+  if (s.few_rows) return run_rows(a, c, residual, m);
   if (s.repack) {
     float* pa = packed != nullptr ? packed : static_cast<float*>(staging(8, (size_t)m * s.k4 * sizeof(float)));
     float* pb = packed != nullptr ? packed + (size_t)m * s.k4
@@ -1358,16 +1427,19 @@ hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, c
   const uint32_t head = s.head_rows;
   const hipError_t e = run(s.plan[0], a, c, residual, head);
   if (e != hipSuccess) return e;
-  return run(s.plan[1], a + (size_t)head * lda, c + (size_t)head * ldc,
-             residual ? residual + (size_t)head * ldr : nullptr, m - head);
+  a += (size_t)head * lda;
+  c += (size_t)head * ldc;
+  if (residual != nullptr) residual += (size_t)head * ldr;
+  return s.tail_rows ? run_rows(a, c, residual, m - head) : run(s.plan[1], a, c, residual, m - head);
 }
 
 uint64_t schedule_partial_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
   if (s.gemv) return 0;
   if (s.few_rows) return s.rows.splits > 1 ? (uint64_t)s.rows.splits * m * n : 0;
   uint64_t need = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * s.head_rows * n : 0;
-  if (s.tail_split && s.plan[1].splits > 1)
-    need = std::max<uint64_t>(need, (uint64_t)s.plan[1].splits * (m - s.head_rows) * n);
+  const int tail_splits = s.tail_rows ? s.rows.splits : s.plan[1].splits;
+  if (s.tail_split && tail_splits > 1)
+    need = std::max<uint64_t>(need, (uint64_t)tail_splits * (m - s.head_rows) * n);
   return need;
 }
 
@@ -1495,8 +1567,8 @@ hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float
     const double tiles = plan_cost(SgemmPlan{4, 1, (int)k}, m, 2 * f, 1);
     if (rows.us < tiles) return launch_sgemm_rows_geglu(rows, a, lda, w, h, ldh, m, f, k, stream);
   }
-  const bool ok = f % 64 == 0 && buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k, (int)k, 4) &&
-                  ldh % 4 == 0 && aligned16(h);
+  const bool ok = f % 64 == 0 && k % kBK == 0 && ldh % 4 == 0 && aligned16(h) &&
+                  buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k);
   if (!ok) return hipErrorNotSupported;
   switch (geglu_height(m)) {
     case 64: launch_geglu_tiles<64>(a, lda, w, h, ldh, m, f, k, stream); break;
@@ -1511,7 +1583,8 @@ hipError_t launch_sgemm_f32_variant(const float* a, const float* b, float* c, ui
   if (tile >= (uint32_t)kVariantTiles || k_slices < 1u || k_slices > 16u) return hipErrorInvalidValue;
   const SgemmPlan p = make_plan((int)tile, (int)k_slices, k);
   const bool aligned = aligned16(a) && aligned16(b);
-  if (p.splits != (int)k_slices || (tile >= 3 && !buffer_path(aligned, (int)k, 0, (int)n, 0, m, n, k, p.k_len, tile)))
+  const bool whole_tiles = k % kBK == 0 || tile == 5 || tile == 6;
+  if (p.splits != (int)k_slices || (tile >= 3 && !(whole_tiles && buffer_path(aligned, (int)k, 0, (int)n, 0, m, n, k))))
     return hipErrorInvalidValue;
   float* partial = nullptr;
   if (p.splits > 1) {
@@ -1566,14 +1639,16 @@ extern "C" PROM_REACTOR_API int prometheus_reactor_sgemm_plan(uint32_t m, uint32
   }
   out_plan->detail_code = PROM_DETAIL_PATH_HIP_MFMA_F32;
   out_plan->estimated_us = s.cost_us;
+  auto report_rows = [&](uint32_t i, uint32_t rows, uint32_t kk) {
+    out_plan->tile_m[i] = (rows + 15u) / 16u * 16u;
+    out_plan->tile_n[i] = (uint32_t)sgemm_rows_columns(s.rows);
+    out_plan->k_slices[i] = (uint32_t)s.rows.splits;
+    out_plan->k_slice_len[i] = s.rows.splits == 1 ? kk : (kk + 15u) / 16u / (uint32_t)s.rows.splits * 16u;
+    out_plan->launches += s.rows.splits > 1 ? 2u : 1u;
+  };
   if (s.few_rows) {
     out_plan->products = 1u;
-    out_plan->tile_m[0] = (m + 15u) / 16u * 16u;
-    out_plan->tile_n[0] = (uint32_t)sgemm_rows_columns(s.rows);
-    out_plan->k_slices[0] = (uint32_t)s.rows.splits;
-    out_plan->k_slice_len[0] = (k + 15u) / 16u / (uint32_t)s.rows.splits * 16u;
-    if (s.rows.splits == 1) out_plan->k_slice_len[0] = k;
-    out_plan->launches = s.rows.splits > 1 ? 2u : 1u;
+    report_rows(0, m, k);
     out_plan->partial_bytes = schedule_partial_floats(s, m, n) * sizeof(float);
     if (has_scratch) out_plan->scratch_bytes = schedule_scratch_floats(s, m, n) * sizeof(float);
     return PROM_OK;
@@ -1586,7 +1661,11 @@ extern "C" PROM_REACTOR_API int prometheus_reactor_sgemm_plan(uint32_t m, uint32
   for (uint32_t i = 0; i < out_plan->products; ++i) {
     const SgemmPlan& p = s.plan[i];
     const uint32_t rows = i == 0 ? s.head_rows : m - s.head_rows;
-    const bool buf = buffer_path(true, (int)kk, 0, ldb_eff, 0, rows, n, kk, p.k_len, p.tile);
+    if (i == 1 && s.tail_rows) {
+      report_rows(1, rows, kk);
+      continue;
+    }
+    const bool buf = buffer_path(true, (int)kk, 0, ldb_eff, 0, rows, n, kk);
     const int tile = (p.tile >= 3 && !buf) ? kStagedFallback[p.tile] : p.tile;
     out_plan->tile_m[i] = (uint32_t)kTileM[tile];
     out_plan->tile_n[i] = (uint32_t)kTileN[tile];
