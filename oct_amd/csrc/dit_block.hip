@@ -23,7 +23,7 @@
 //   resid_norm_mod r = x + gateA * RMSNorm(proj; n2)             -> fp32
 //                  f = RMSNorm(r; n3) * scaleM                   -> bf16
 //   swiglu         h = silu(g) * u -> bf16, fused into the W1|W3 GEMM epilogue
-//                  (gemm_bf16.hip) when F % 128 == 0 and D % 64 == 0
+//                  (gemm_bf16.hip, gemm_bf16_tiles.hip) when F % 8 == 0
 //   (W2 GEMM       -> bf16 w2)
 //   final_resid    out = r + gateM * RMSNorm(w2; n4)              -> fp32
 // The bf16 intermediates (qkv, proj, w2) are each normalised before they
@@ -353,12 +353,14 @@ hipError_t enqueue_dit(const PrometheusDitBlockBf16Request* r, char* ws, const s
   // CU as well) took three, the last with 16 (45 -> 37.5 us).  R is next read
   // after the FFN GEMMs and the block output by the next block's first
   // kernel: both go out as streaming stores (W1|W3 -4 us, the first row
-  // kernel -1.3, this one -1.2).
-  hipLaunchKernelGGL((rows::resid_norm_mod_kernel<uint16_t, 12, uint16_t, true>), rows::row_groups<12>(T), dim3(768), 0, st, r->input, projb, r->attn_norm2, gateA, r->ffn_norm1, scaleM,
-                     R, Fb, T, D, eps, f_slice);
+  // kernel -1.3, this one -1.2).  (Four rows per workgroup also at few
+  // tokens: 235 us against 233 for the block at T = 288.)
+  hipLaunchKernelGGL((rows::resid_norm_mod_kernel<uint16_t, 12, uint16_t, true>), rows::row_groups<12>(T),
+                     dim3(768), 0, st, r->input, projb, r->attn_norm2, gateA, r->ffn_norm1, scaleM, R, Fb, T, D, eps,
+                     f_slice);
   PROM_STEP(hipGetLastError());
   // FFN up-projection with SwiGLU fused into the GEMM epilogue when the shape
-  // allows (F a multiple of 128, D of 64); otherwise GEMM to fp32, then SwiGLU.
+  // allows (F a multiple of 8); otherwise GEMM to fp32, then SwiGLU.
   // (G, unused on the fused path, takes the K-slice sums of a final partial wave.)
   uint32_t k13 = 1;
   const hipError_t fused =
