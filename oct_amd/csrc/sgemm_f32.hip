@@ -1133,11 +1133,14 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
   // The eight-wave 128x128 kernel is tried first and is only replaced by a
   // plan more than 1 % cheaper (near ties keep the established kernel; the
   // model is accurate to a few per cent).
-  static const int kTileOrder[kTileShapes] = {4, 3, 0, 1, 2, 5, 6, 7};
+  static const int kTileOrder[kTileShapes + 1] = {4, 3, 0, 1, 2, 5, 6, 7, 4};
   const Rows kind = operand_rows(aligned, lda, sa, ldb, sb, m, n, k);
   SgemmPlan best = make_plan(0, 1, k);
   double best_cost = 1e300;
-  for (int t : kTileOrder) {
+  for (int i = 0; i <= kTileShapes; ++i) {
+    const int t = kTileOrder[i];
+    const bool last = i == kTileShapes;
+    if (last && k % kBK == 0) break;
     for (int s : kSplitChoices) {
       if (s > 1 && (batch > 1 || k / (uint32_t)s < 64)) break;
       if (s > 1 && t == 7) break;  // sliced, 64x128 measured within 2 % of the other tiles
@@ -1146,8 +1149,10 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
       if (p.splits > 1 && (uint64_t)p.splits * m * n > max_partial_floats) continue;
       if (t >= 3 && !buffer_path(aligned, lda, sa, ldb, sb, m, n, k)) continue;
       // K tails: the 64x64 tiles, and 128x128, whose offsets (to a K tile past B) stay
-      // below 2^32 if B has a K tile itself
-      if ((t == 3 || t == 7 || (t == 4 && k < (uint32_t)kBK)) && k % kBK != 0) continue;
+      // below 2^32 if B has a K tile itself.  Unsliced, as slices of tall products would
+      // need more scratch than the allocation-free entry has, and as the last
+      // candidate, so that among the others the choice is as without it.
+      if (k % kBK != 0 && (t == 3 || t == 7 || (t == 4 && (s > 1 || !last || k < (uint32_t)kBK)))) continue;
       const double c = plan_cost(p, m, n, batch, kind);
       if (c < best_cost * 0.99) {
         best_cost = c;
@@ -1316,7 +1321,14 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
     const bool tail_rows = k < 1024u && few_rows_win(tail, n, k, lda, ldb, tail_us, max_partial_floats, &rows);
     if (tail_rows) tail_us = rows.us;
     const double split_cost = plan_cost(ph, head, n, 1, kind) + tail_us;
-    if (split_cost < s.cost_us) {
+    // (of unaligned operands' slices, those that the allocation-free entry can hold)
+    const uint64_t limit = PROM_SGEMM_NOALLOC_SCRATCH_BYTES / sizeof(float);
+    const uint64_t whole = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * m * n : 0;
+    const uint64_t in_head = ph.splits > 1 ? (uint64_t)ph.splits * head * n : 0;
+    const int tail_splits = tail_rows ? rows.splits : pt.splits;
+    const uint64_t in_tail = tail_splits > 1 ? (uint64_t)tail_splits * tail * n : 0;
+    const bool only_split_fits = kind != Rows::kAligned && whole > limit && std::max(in_head, in_tail) <= limit;
+    if (split_cost < s.cost_us || only_split_fits) {
       s.tail_split = true;
       s.tail_rows = tail_rows;
       if (tail_rows) s.rows = rows;
@@ -1327,6 +1339,26 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
     }
   }
   return s;
+}
+
+uint64_t schedule_repack_floats(const SgemmSchedule& s, uint32_t m) {
+  return s.repack ? (uint64_t)m * s.k4 + (uint64_t)s.k4 * s.n4 : 0;
+}
+
+uint64_t schedule_partial_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
+  if (s.gemv) return 0;
+  if (s.few_rows) return s.rows.splits > 1 ? (uint64_t)s.rows.splits * m * n : 0;
+  uint64_t need = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * s.head_rows * n : 0;
+  const int tail_splits = s.tail_rows ? s.rows.splits : s.plan[1].splits;
+  if (s.tail_split && tail_splits > 1)
+    need = std::max<uint64_t>(need, (uint64_t)tail_splits * (m - s.head_rows) * n);
+  return need;
+}
+
+// Floats of scratch the schedule needs in one array: the split-K partials
+// rounded up to 256 bytes, then the padded copies of A and B.
+uint64_t schedule_scratch_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
+  return ((schedule_partial_floats(s, m, n) + 63) & ~63ull) + schedule_repack_floats(s, m);
 }
 
 SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_t n, uint32_t k, bool has_residual,
@@ -1346,15 +1378,22 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
   if (!direct) {
     const uint32_t k4 = (k + 3u) & ~3u, n4 = (n + 3u) & ~3u;
     if ((size_t)(m + 128) * k4 * 4 < (1ull << 31) && ((size_t)k4 * n4 + 256) * 4 < (1ull << 31)) {
-      SgemmSchedule r = schedule_products(true, (int)k4, (int)n4, m, n, k4, max_partial_floats);
+      // where the copies fit the allocation-free entry's scratch, what is sliced fits
+      // beside them
+      const uint64_t limit = PROM_SGEMM_NOALLOC_SCRATCH_BYTES / sizeof(float);
+      const uint64_t copies = (uint64_t)m * k4 + (uint64_t)k4 * n4;
+      const uint64_t beside =
+          copies + 64 <= limit ? std::min(max_partial_floats, limit - copies - 64) : max_partial_floats;
+      SgemmSchedule r = schedule_products(true, (int)k4, (int)n4, m, n, k4, beside);
       const double bytes = 4.0 * ((double)m * k + (double)k * n + (double)m * k4 + (double)k4 * n4);
       r.cost_us += 4.0 + bytes / 3.0e6;
-      if (r.cost_us < s.cost_us) {
-        r.repack = true;
-        r.k4 = k4;
-        r.n4 = n4;
-        s = r;
-      }
+      r.repack = true;
+      r.k4 = k4;
+      r.n4 = n4;
+      // slices that it cannot hold give way to copies that it can
+      const bool only_copies_fit =
+          schedule_scratch_floats(s, m, n) > limit && schedule_scratch_floats(r, m, n) <= limit;
+      if (r.cost_us < s.cost_us || only_copies_fit) s = r;
     }
   }
   SgemmRowsPlan rows;
@@ -1366,10 +1405,6 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
     s.cost_us = rows.us;
   }
   return s;
-}
-
-uint64_t schedule_repack_floats(const SgemmSchedule& s, uint32_t m) {
-  return s.repack ? (uint64_t)m * s.k4 + (uint64_t)s.k4 * s.n4 : 0;
 }
 
 // Queues schedule s; partial (null: runtime staging slot 6) receives the
@@ -1431,22 +1466,6 @@ hipError_t run_sgemm_schedule(const SgemmSchedule& s, const float* a, int lda, c
   c += (size_t)head * ldc;
   if (residual != nullptr) residual += (size_t)head * ldr;
   return s.tail_rows ? run_rows(a, c, residual, m - head) : run(s.plan[1], a, c, residual, m - head);
-}
-
-uint64_t schedule_partial_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
-  if (s.gemv) return 0;
-  if (s.few_rows) return s.rows.splits > 1 ? (uint64_t)s.rows.splits * m * n : 0;
-  uint64_t need = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * s.head_rows * n : 0;
-  const int tail_splits = s.tail_rows ? s.rows.splits : s.plan[1].splits;
-  if (s.tail_split && tail_splits > 1)
-    need = std::max<uint64_t>(need, (uint64_t)tail_splits * (m - s.head_rows) * n);
-  return need;
-}
-
-// Floats of scratch the schedule needs in one array: the split-K partials
-// rounded up to 256 bytes, then the padded copies of A and B.
-uint64_t schedule_scratch_floats(const SgemmSchedule& s, uint32_t m, uint32_t n) {
-  return ((schedule_partial_floats(s, m, n) + 63) & ~63ull) + schedule_repack_floats(s, m);
 }
 
 }  // namespace

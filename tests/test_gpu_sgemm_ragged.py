@@ -82,3 +82,14 @@ def test_ragged_plans_fit_their_report(m, n, k):
     kk = (k + 3) // 4 * 4 if info.repacked else k
     for i in range(info.products):
         assert info.k_slices[i] == 1 or info.k_slice_len[i] * info.k_slices[i] >= kk - 16 * info.k_slices[i]
+
+
+@pytest.mark.parametrize("m,n,k", [(14050, 976, 6828), (2109, 1518, 3169), (5722, 4096, 1581), (168, 11520, 6074),
+                                   (3496, 4276, 11340), (620, 2527, 3414), (8192, 4784, 8200)])
+def test_ragged_plans_stay_within_the_noalloc_scratch(m, n, k):
+    """Tall products with K tails and unaligned rows that have a plan within the
+    allocation-free entry's scratch take one."""
+    info = p.PrometheusSgemmPlanInfo()
+    info.struct_size = ctypes.sizeof(info)
+    assert p.shared_library().prometheus_reactor_sgemm_plan(m, n, k, ctypes.byref(info)) == p.PROM_OK
+    assert info.scratch_bytes <= p.SGEMM_NOALLOC_SCRATCH_BYTES
