@@ -63,8 +63,9 @@ constexpr uint64_t kRuntimeMagic = 0x4F43544D49333535ull;  // "OCTMI355"
 constexpr uint32_t kEventSlots = 64;
 // Staging slots: 0-3 operand staging, 4 block workspace, 5 block host staging,
 // 6 split-K partials, 7 FFT twiddle table, 8-9 padded GEMM operand copies,
-// 10 row-reduction parts.
+// 10 row-reduction parts (had from the start, so that a reduction allocates nothing).
 constexpr uint32_t kStagingSlots = 11;
+constexpr size_t kRowPartsBytes = 2u << 20;
 
 struct AsyncState;  // async task table, submission slots and batch arenas (sgemm_async.hip)
 struct ModelState;  // resident model block and compiled session (model_block.hip)

@@ -335,15 +335,26 @@ hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, f
                        uint32_t width, uint32_t stride, float eps, hipStream_t stream) {
   if (p.waves == 0) {
     const uint32_t n = (width + kPartValues - 1) / kPartValues;
-    RowPart* parts = static_cast<RowPart*>(staging(10, (size_t)rows * n * sizeof(RowPart)));
+    // The parts' buffer is had with the device; more rows than it holds the parts of go
+    // in blocks, one after the other on the stream (2^17 parts are 2^30 values).
+    const uint32_t block = std::max(1u, (uint32_t)(kRowPartsBytes / sizeof(RowPart)) / n);
+    RowPart* parts = static_cast<RowPart*>(staging(10, std::max(kRowPartsBytes, (size_t)n * sizeof(RowPart))));
     if (parts == nullptr) return hipErrorOutOfMemory;
-    hipLaunchKernelGGL((row_parts_kernel<kOp>), dim3(rows * n), dim3(256), 0, stream, in, parts, n, width, stride);
-    const hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    const uint32_t blocks = kOp == kOpSum || kOp == kOpMax ? (rows + 3u) / 4u : rows * n;
-    hipLaunchKernelGGL((row_finish_kernel<kOp>), dim3(blocks), dim3(256), 0, stream, in, w, out, aux, parts, n, rows,
-                       width, stride, eps);
-    return hipGetLastError();
+    constexpr bool kScalar = kOp == kOpSum || kOp == kOpMax;
+    for (uint32_t r = 0; r < rows; r += std::min(block, rows - r)) {
+      const uint32_t count = std::min(block, rows - r);
+      const float* x = in + (size_t)r * stride;
+      hipLaunchKernelGGL((row_parts_kernel<kOp>), dim3(count * n), dim3(256), 0, stream, x, parts, n, width, stride);
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+      const uint32_t blocks = kScalar ? (count + 3u) / 4u : count * n;
+      hipLaunchKernelGGL((row_finish_kernel<kOp>), dim3(blocks), dim3(256), 0, stream, x, w,
+                         out + (kScalar ? r : (size_t)r * width), aux != nullptr ? aux + r : nullptr, parts, n, count,
+                         width, stride, eps);
+      const hipError_t e2 = hipGetLastError();
+      if (e2 != hipSuccess) return e2;
+    }
+    return hipSuccess;
   }
 #define ROWS(W, C)                                                                                                   \
   hipLaunchKernelGGL((row_kernel<kOp, W, C, kTail>), dim3(W == 1 ? (rows + 3u) / 4u : rows),                         \

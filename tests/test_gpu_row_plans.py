@@ -108,3 +108,28 @@ def test_infinities_and_nan(gpu_runtime, width):
     s = reduce_on_device(gpu_runtime, x, p.OP_SUM)
     assert s[0] == -np.inf and s[1] == -np.inf and np.isnan(s[2]) and np.isnan(s[3])
     assert s[4] == np.inf and s[5] == -np.inf
+
+
+@pytest.mark.parametrize("op", [p.OP_SUM, p.OP_SOFTMAX])
+def test_more_parts_than_the_buffer_holds(gpu_runtime, op):
+    """26220 rows of 5 parts each go in blocks of 2^17 // 5 = 26214 rows."""
+    rt, rows, width = gpu_runtime, 26220, 32769
+    picks = [0, 26213, 26214, 26219]
+    d = Device(rt, 0)
+    src = d.new(rows * width)
+    dst = d.new(rows * width if op == p.OP_SOFTMAX else rows)
+    x = oracle.normal(5, (len(picks), width))
+    for i, row in enumerate(picks):
+        rt.upload(src + 4 * row * width, x[i])
+    rt.reduction_device(src, dst, rows, width, op)
+    for i, row in enumerate(picks):
+        v = x[i].astype(np.float64)
+        if op == p.OP_SUM:
+            want, got, ulps = np.array([v.sum()]), d.get(dst + 4 * row, (1,)), 8.0
+        else:
+            # x - max and its product with log2 e round once each, and the power takes
+            # both errors, |x - max| half ulps each, as relative ones
+            e = np.exp(v - v.max())
+            want, got, ulps = e / e.sum(), d.get(dst + 4 * row * width, (width,)), 8 + 2 * np.abs(v - v.max())
+        assert np.all(np.abs(got - want) <= ulps * 2.0 ** -24 * np.abs(want) + 1e-37), row
+    d.free()
