@@ -605,12 +605,12 @@ enum class Bf16Path { kFiveStage, kTiles, kPadded, kSmall };
 // more than the register-staged kernel's 16-bit loads (about 5.5 us per K tile of
 // 64 there: 1023x2049x777 82 us, 33x3001x5003 324 us).
 Bf16Path bf16_path(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n, uint32_t k,
-                   Bf16TilePlan* plan) {
+                   Bf16TilePlan* plan, bool blocked) {
   *plan = plan_bf16_tiles(m, n, k, false);
   if (bf16_tiles_take(a, lda, b, ldb, k)) {
     const bool range = (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * ldb * 2 < (1ull << 31);
-    return range && k % kBK4 == 0 && bf16_five_stage_us(m, n, k, 0) < plan->us ? Bf16Path::kFiveStage
-                                                                                  : Bf16Path::kTiles;
+    const double five_us = bf16_five_stage_us(m, n, k, 0) * (blocked ? 0.965 : 1.0);
+    return range && k % kBK4 == 0 && five_us < plan->us ? Bf16Path::kFiveStage : Bf16Path::kTiles;
   }
   if (k >= (1u << 22) - 8 || n >= (1u << 23) - 8) return Bf16Path::kSmall;
   const double tiles128 = (double)((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
@@ -657,7 +657,7 @@ bool blocked_range(int a_slice, uint32_t m, uint32_t k) {
 bool gemm_bf16_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n,
                                uint32_t k) {
   Bf16TilePlan plan;
-  return bf16_path(a, lda, b, ldb, m, n, k, &plan) == Bf16Path::kFiveStage;
+  return bf16_path(a, lda, b, ldb, m, n, k, &plan, true) == Bf16Path::kFiveStage;
 }
 
 bool gemm_bf16_swiglu_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f,
@@ -669,7 +669,7 @@ hipError_t launch_gemm_bf16_ex(const uint16_t* a, int lda, const uint16_t* b, in
                                int ldc, uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr,
                                hipStream_t stream, int* path_detail, int a_slice) {
   Bf16TilePlan plan;
-  Bf16Path path = bf16_path(a, lda, b, ldb, m, n, k, &plan);
+  Bf16Path path = bf16_path(a, lda, b, ldb, m, n, k, &plan, a_slice > 0);
   if (a_slice > 0 && (path != Bf16Path::kFiveStage || !blocked_range(a_slice, m, k))) return hipErrorNotSupported;
   if (path_detail) *path_detail = PROM_DETAIL_PATH_HIP_MFMA_BF16;
   if (path == Bf16Path::kFiveStage) {
