@@ -134,13 +134,27 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
           if (k0 + 4 * grp + c >= p.k) q.a[mb][c] = 0.0f;
     }
   };
-  floatx4 acc[kH][kMB][kC];
+  // Sums of four granules (64 of k) at a time go into `total`: a chain of 64 and one of
+  // the blocks, whose rounding is that of the tiles' K slices or less where one chain
+  // over a long K has more (13x9344x7680: 5.6e-7 of the result, the tiles 3.3e-7).
+  floatx4 acc[kH][kMB][kC], total[kH][kMB][kC];
 #pragma unroll
   for (int h = 0; h < kH; ++h)
 #pragma unroll
     for (int mb = 0; mb < kMB; ++mb)
 #pragma unroll
-      for (int j = 0; j < kC; ++j) acc[h][mb][j] = floatx4{};
+      for (int j = 0; j < kC; ++j) acc[h][mb][j] = total[h][mb][j] = floatx4{};
+  auto add_up = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int h = 0; h < kH; ++h)
+#pragma unroll
+      for (int mb = 0; mb < kMB; ++mb)
+#pragma unroll
+        for (int j = 0; j < kC; ++j) {
+          total[h][mb][j] += acc[h][mb][j];
+          acc[h][mb][j] = floatx4{};
+        }
+  };
   auto compute = [&](const Granule& q) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < 4; ++c)
@@ -159,13 +173,15 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
   Granule q;
   int g = g0 + wave;
   if (g < g1) load(q, g);
-  for (; g + kW < g1; g += kW) {
+  for (int done = 1; g + kW < g1; g += kW, ++done) {
     Granule next;
     load(next, g + kW);
     compute(q);
+    if ((done & 3) == 0) add_up();
     q = next;
   }
   if (g < g1) compute(q);
+  add_up();
 
   // D[i][j] is in lane j + 16 (i / 4), register i % 4; block j of a half holds its
   // columns kC * (lane % 16) + j.
@@ -177,7 +193,7 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
       for (int j = 0; j < kC; ++j)
 #pragma unroll
         for (int i = 0; i < 4; ++i)
-          sums[wave][((h * 16 * kMB) + 16 * mb + 4 * grp + i) * kCols + kC * li + j] = acc[h][mb][j][i];
+          sums[wave][((h * 16 * kMB) + 16 * mb + 4 * grp + i) * kCols + kC * li + j] = total[h][mb][j][i];
   __syncthreads();
   float* out = p.c + (gridDim.y > 1 ? blockIdx.y * p.slab : 0);
   for (int e = tid; e < 16 * kMB * kCols; e += 64 * kW) {
