@@ -164,7 +164,9 @@ __global__ __launch_bounds__(256) void pinned_copy_kernel(const uint4* __restric
 
 // A ring of kSlots pinned slots.  take() hands out consecutive regions of the
 // current slot; a slot is left with an event behind its last copy and entered
-// again only once that event has passed.
+// again only once that event has passed.  The event covers what is queued when
+// take() leaves the slot, so the copies of every region taken before have to be
+// queued by then: pieces that are filled together are parts of one region.
 struct Ring {
   size_t slot_bytes = 0;
   bool tried = false, ready = false;
@@ -191,20 +193,22 @@ struct Ring {
     ready = true;
     return true;
   }
-  // `bytes` <= slot_bytes for a copy on st; null: *e says why.
+  // `bytes` <= slot_bytes for copies on st; null: *e says why, and the ring stays in
+  // its slot.
   char* take(size_t bytes, hipStream_t st, hipError_t* e) {
     *e = hipSuccess;
     if (used > 0 && (st != stream || used + bytes > slot_bytes)) {
       *e = hipEventRecord(done[current], stream);
       if (*e != hipSuccess) return nullptr;
       busy[current] = true;
-      current = (current + 1) % kSlots;
-      used = 0;
-      if (busy[current]) {
-        *e = hipEventSynchronize(done[current]);
+      const int next = (current + 1) % kSlots;
+      if (busy[next]) {
+        *e = hipEventSynchronize(done[next]);
         if (*e != hipSuccess) return nullptr;
-        busy[current] = false;
+        busy[next] = false;
       }
+      current = next;
+      used = 0;
     }
     stream = st;
     char* p = slot[current] + used;
@@ -277,19 +281,18 @@ hipError_t upload_host(void* dst, const void* src, size_t bytes, hipStream_t str
   if (ring == nullptr) return hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream);
   const char* s8 = static_cast<const char*>(src);
   char* d8 = static_cast<char*>(dst);
-  // A copy of two small pieces is one job; larger ones go piece by piece, so that no
-  // piece waits for a slot before its turn.
-  const int most = bytes <= 2 * piece && piece < kKernelMax ? 2 : 1;
+  // A copy of two pieces below 4 MiB is one job in one region of a slot; larger ones go
+  // piece by piece, so that no piece waits for a slot before its turn.
+  const size_t region = bytes <= 2 * piece && piece < kKernelMax ? bytes : piece;
   for (size_t off = 0; off < bytes;) {
+    const size_t all = std::min(region, bytes - off);
+    hipError_t e;
+    char* const pinned = ring->take(all, stream, &e);
+    if (pinned == nullptr) return e;
     CopyPool::Piece job[2];
     int n = 0;
-    for (size_t at = off; n < most && at < bytes; at += piece, ++n) {
-      const size_t len = std::min(piece, bytes - at);
-      hipError_t e;
-      char* pinned = ring->take(len, stream, &e);
-      if (pinned == nullptr) return e;
-      job[n] = {pinned, s8 + at, len};
-    }
+    for (size_t at = 0; at < all; at += piece, ++n)
+      job[n] = {pinned + at, s8 + off + at, std::min(piece, all - at)};
     p.pool.begin(job, n);
     hipError_t first = hipSuccess;
     for (int c = 0; c < n; ++c) {
@@ -324,7 +327,8 @@ hipError_t download_host(void* dst, const void* src, size_t bytes, hipStream_t s
     return e;
   }
   // Up to kSlots pieces are queued ahead of the host copies; piece i is copied out
-  // before piece i + kSlots is queued, so no piece's region is taken again early.
+  // before piece i + kSlots is queued, so no piece's region is taken again early, and
+  // each piece's move is queued before the next region is taken.
   const size_t chunks = (bytes + piece - 1) / piece;
   char* pinned[kSlots] = {};
   auto length = [&](size_t i) { return std::min(piece, bytes - i * piece); };

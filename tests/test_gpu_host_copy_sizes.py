@@ -39,3 +39,18 @@ def test_slots_are_reused_with_fresh_data(gpu_runtime):
         b = np.full((k, n), np.float32(1 + i % 3))
         out, _ = gpu_runtime.sgemm(m, n, k, a, b)
         assert np.all(np.asarray(out) == np.float32((i + 1) * (1 + i % 3) * k))
+
+
+def test_batch_uploads_run_ahead_of_the_device(gpu_runtime):
+    """A batch queues its uploads, products and downloads without a wait between them: operands
+    of 1 to 8 MiB, which leave a slot in the middle, and 20 MiB, which come round the ring."""
+    shapes = [(75, 975, 2048), (320, 64, 4096), (16, 1280, 4096), (300, 300, 1000), (64, 2000, 975)]
+    problems = []
+    for i in range(48):
+        m, n, k = shapes[i % len(shapes)]
+        problems.append((np.full((m, k), np.float32(i + 1)), np.full((k, n), np.float32(1 + i % 3))))
+    rc, status, outs = gpu_runtime.sgemm_batch(problems)
+    assert rc == 0, status
+    for i, (out, (a, _)) in enumerate(zip(outs, problems)):
+        # every partial sum is a whole number below 2^24: exact in any order
+        assert np.all(out == np.float32((i + 1) * (1 + i % 3) * a.shape[1])), i
