@@ -1281,14 +1281,28 @@ struct SgemmSchedule {
   double cost_us;      // plan-model estimate of the queued work
 };
 
+// The allocation-free entry's scratch.  Its plan is the allocating entry's, so a plan
+// that outgrows the array is a call refused: where one that fits is estimated within 2 %
+// (the models' own error is larger) it is taken, in the cases marked below.  Elsewhere
+// the fastest plan stands and the entry refuses it (1280x2048x8192: 80 MiB of slices).
+constexpr uint64_t kNoallocFloats = PROM_SGEMM_NOALLOC_SCRATCH_BYTES / sizeof(float);
+constexpr double kFitsWithin = 1.02;
+
+uint64_t sliced_floats(int splits, uint32_t m, uint32_t n) { return splits > 1 ? (uint64_t)splits * m * n : 0; }
+
 // Whether the few-rows kernel takes an m x n x k product that the tiles are estimated
 // to run in tiles_us.  The two models meet where both are off: a sliced product of a
 // small B measured slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger
-// one faster (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
+// one faster (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).  Slices that
+// outgrow the allocation-free scratch (45x67176x7772: 6, 69 MiB) give way to fewer.
 bool few_rows_win(uint32_t m, uint32_t n, uint32_t k, int lda, int ldb, double tiles_us, uint64_t max_partial_floats,
                   SgemmRowsPlan* rows) {
   if (!sgemm_rows_take(m, k, lda, ldb, 1)) return false;
   *rows = plan_sgemm_rows(m, n, k, false, max_partial_floats);
+  if (sliced_floats(rows->splits, m, n) > kNoallocFloats) {
+    const SgemmRowsPlan fits = plan_sgemm_rows(m, n, k, false, std::min(max_partial_floats, kNoallocFloats));
+    if (fits.us <= kFitsWithin * rows->us) *rows = fits;
+  }
   const bool small = (uint64_t)n * k < (1u << 20);
   const double bias = small ? (rows->splits > 1 ? 1.6 : 0.0) : -0.06 * tiles_us;
   return rows->us + bias < tiles_us;
@@ -1301,7 +1315,18 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
   SgemmSchedule s{};
   s.head_rows = m;
   const Rows kind = operand_rows(aligned, lda, 0, ldb, 0, m, n, k);
-  s.plan[0] = plan_sgemm(aligned, lda, 0, ldb, 0, m, n, k, 1, max_partial_floats);
+  // The plan of `rows` rows; slices of unaligned operands, which cost less than predicated
+  // loads would, keep to the allocation-free scratch (49370x33x6182: 8, not 12 of 75 MiB).
+  auto plan_rows = [&](bool rows_aligned, uint32_t rows, uint64_t max_floats) {
+    SgemmPlan p = plan_sgemm(rows_aligned, lda, 0, ldb, 0, rows, n, k, 1, max_floats);
+    if (kind != Rows::kAligned && sliced_floats(p.splits, rows, n) > kNoallocFloats) {
+      const SgemmPlan fits =
+          plan_sgemm(rows_aligned, lda, 0, ldb, 0, rows, n, k, 1, std::min(max_floats, kNoallocFloats));
+      if (plan_cost(fits, rows, n, 1, kind) <= kFitsWithin * plan_cost(p, rows, n, 1, kind)) p = fits;
+    }
+    return p;
+  };
+  s.plan[0] = plan_rows(aligned, m, max_partial_floats);
   s.cost_us = plan_cost(s.plan[0], m, n, 1, kind);
   // A partial last row of 128-row tiles runs nearly empty for the whole K depth
   // (M = 1056: a 32-row tail in 9 tile rows).  When the estimate favours it, the
@@ -1312,30 +1337,46 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
   if (tail != 0 && m > 128u) {
     const uint32_t head = m - tail;
     const bool tail_aligned = aligned && (lda % 4 == 0);
-    const SgemmPlan ph = plan_sgemm(aligned, lda, 0, ldb, 0, head, n, k, 1, max_partial_floats);
-    const SgemmPlan pt = plan_sgemm(tail_aligned, lda, 0, ldb, 0, tail, n, k, 1, max_partial_floats);
-    double tail_us = plan_cost(pt, tail, n, 1, kind);
-    // The few-rows kernel takes short K's tails, which the tiles cannot slice (one row
-    // of 3001x516: 5.5 us against 10); a long K's are 1 or 2 % of the whole either way.
-    SgemmRowsPlan rows;
-    const bool tail_rows = k < 1024u && few_rows_win(tail, n, k, lda, ldb, tail_us, max_partial_floats, &rows);
-    if (tail_rows) tail_us = rows.us;
-    const double split_cost = plan_cost(ph, head, n, 1, kind) + tail_us;
+    struct TailSplit {
+      SgemmPlan head, tail;
+      SgemmRowsPlan rows;
+      bool tail_rows;
+      double us;
+      uint64_t partial_floats;
+    };
+    auto plan_split = [&](uint64_t max_floats) {
+      TailSplit q{};
+      q.head = plan_rows(aligned, head, max_floats);
+      q.tail = plan_rows(tail_aligned, tail, max_floats);
+      double tail_us = plan_cost(q.tail, tail, n, 1, kind);
+      // The few-rows kernel takes short K's tails, which the tiles cannot slice (one row
+      // of 3001x516: 5.5 us against 10); a long K's are 1 or 2 % of the whole either way.
+      q.tail_rows = k < 1024u && few_rows_win(tail, n, k, lda, ldb, tail_us, max_floats, &q.rows);
+      if (q.tail_rows) tail_us = q.rows.us;
+      q.us = plan_cost(q.head, head, n, 1, kind) + tail_us;
+      q.partial_floats = std::max(sliced_floats(q.head.splits, head, n),
+                                  sliced_floats(q.tail_rows ? q.rows.splits : q.tail.splits, tail, n));
+      return q;
+    };
+    TailSplit q = plan_split(max_partial_floats);
+    const uint64_t whole = sliced_floats(s.plan[0].splits, m, n);
+    // A whole product that fits the allocation-free scratch is not split into slices that
+    // do not (1133x19688x16612: eight slices of its 109-row tail are 65 MiB).
+    if (whole <= kNoallocFloats && q.partial_floats > kNoallocFloats) {
+      const TailSplit fits = plan_split(std::min(max_partial_floats, kNoallocFloats));
+      if (std::min(fits.us, s.cost_us) <= kFitsWithin * q.us) q = fits;
+    }
     // (of unaligned operands' slices, those that the allocation-free entry can hold)
-    const uint64_t limit = PROM_SGEMM_NOALLOC_SCRATCH_BYTES / sizeof(float);
-    const uint64_t whole = s.plan[0].splits > 1 ? (uint64_t)s.plan[0].splits * m * n : 0;
-    const uint64_t in_head = ph.splits > 1 ? (uint64_t)ph.splits * head * n : 0;
-    const int tail_splits = tail_rows ? rows.splits : pt.splits;
-    const uint64_t in_tail = tail_splits > 1 ? (uint64_t)tail_splits * tail * n : 0;
-    const bool only_split_fits = kind != Rows::kAligned && whole > limit && std::max(in_head, in_tail) <= limit;
-    if (split_cost < s.cost_us || only_split_fits) {
+    const bool only_split_fits =
+        kind != Rows::kAligned && whole > kNoallocFloats && q.partial_floats <= kNoallocFloats;
+    if (q.us < s.cost_us || only_split_fits) {
       s.tail_split = true;
-      s.tail_rows = tail_rows;
-      if (tail_rows) s.rows = rows;
+      s.tail_rows = q.tail_rows;
+      if (q.tail_rows) s.rows = q.rows;
       s.head_rows = head;
-      s.plan[0] = ph;
-      s.plan[1] = pt;
-      s.cost_us = split_cost;
+      s.plan[0] = q.head;
+      s.plan[1] = q.tail;
+      s.cost_us = q.us;
     }
   }
   return s;
@@ -1380,7 +1421,7 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
     if ((size_t)(m + 128) * k4 * 4 < (1ull << 31) && ((size_t)k4 * n4 + 256) * 4 < (1ull << 31)) {
       // where the copies fit the allocation-free entry's scratch, what is sliced fits
       // beside them
-      const uint64_t limit = PROM_SGEMM_NOALLOC_SCRATCH_BYTES / sizeof(float);
+      const uint64_t limit = kNoallocFloats;
       const uint64_t copies = (uint64_t)m * k4 + (uint64_t)k4 * n4;
       const uint64_t beside =
           copies + 64 <= limit ? std::min(max_partial_floats, limit - copies - 64) : max_partial_floats;

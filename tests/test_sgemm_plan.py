@@ -157,3 +157,16 @@ def test_plan_accepts_the_struct_without_scratch_bytes():
     assert bytes(buf[short:]) == b"\xab" * (len(buf) - short)
     info.struct_size = short - 1
     assert lib.prometheus_reactor_sgemm_plan(4, 4, 4, ctypes.byref(info)) == p.PROM_ERROR
+
+
+@pytest.mark.parametrize("m,n,k", [
+    # a tail of rows whose K slices would outgrow the array where the whole product needs none
+    (1133, 19688, 16612), (3070, 16808, 5572), (2418, 12480, 9172), (7790, 19432, 18760), (3583, 27108, 3312),
+    (722, 28080, 5104),
+    # few rows against a wide matrix, tall products with unaligned rows
+    (45, 67176, 7772), (37, 116590, 4352), (48, 50880, 9708), (49370, 33, 6182), (156696, 31, 3257)])
+def test_products_with_a_plan_within_the_noalloc_scratch_take_it(m, n, k):
+    """Each has a plan within the allocation-free entry's array that is estimated within
+    2 % of the fastest, so that entry takes it."""
+    rc, i = _plan(m, n, k)
+    assert rc == p.PROM_OK and i.scratch_bytes <= p.SGEMM_NOALLOC_SCRATCH_BYTES
