@@ -1049,14 +1049,15 @@ SgemmPlan make_plan(int tile, int splits, uint32_t k) {
 }
 
 // True when the direct-to-LDS kernels apply: operands of 16-byte aligned rows and
-// every 32-bit byte offset (rows up to M + 192, all of B plus a tile row) in range.
+// every 32-bit byte offset (rows up to M + 128, all of B plus a tile row) in range; the
+// 192-row GeGLU tile is the only one of its column, for more than 128 rows (geglu_height).
 // `aligned`: both operand base addresses are 16-byte aligned.  A K tail (k % 4 == 0)
 // is taken in the last tile of the last slice (by tiles 4, 5 and 6).
 bool buffer_path(bool aligned, int lda, long long sa, int ldb, long long sb, uint32_t m, uint32_t n, uint32_t k) {
   // B chunks past column n lie in B's padding or next row and only feed
   // output columns that are never stored, so n itself may be ragged.
   const bool vec = (k % 4 == 0) && (lda % 4 == 0) && (ldb % 4 == 0) && (sa % 4 == 0) && (sb % 4 == 0) && aligned;
-  return vec && (size_t)(m + 192) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
+  return vec && (size_t)(m + 128) * lda * 4 < (1ull << 31) && ((size_t)k * ldb + n + 256) * 4 < (1ull << 31);
 }
 
 // True when the register-staged kernels read through buffer descriptors: every 32-bit

@@ -170,3 +170,11 @@ def test_products_with_a_plan_within_the_noalloc_scratch_take_it(m, n, k):
     2 % of the fastest, so that entry takes it."""
     rc, i = _plan(m, n, k)
     assert rc == p.PROM_OK and i.scratch_bytes <= p.SGEMM_NOALLOC_SCRATCH_BYTES
+
+
+@pytest.mark.parametrize("m,n,k", [(17996, 2996, 29656), (18406, 7724, 29088), (19351, 84, 27504)])
+def test_operands_up_to_128_rows_below_2_gib_run_direct(m, n, k):
+    """The direct-to-LDS tiles address A with 32-bit byte offsets, up to a tile's 128 rows past it."""
+    rc, i = _plan(m, n, k)
+    assert (m - m % 128 + 128) * k * 4 < 2**31 < (m + 192) * k * 4
+    assert rc == p.PROM_OK and all(i.direct_to_lds[:i.products])
