@@ -1420,21 +1420,28 @@ SgemmSchedule schedule_sgemm(bool aligned, int lda, int ldb, uint32_t m, uint32_
   if (!direct) {
     const uint32_t k4 = (k + 3u) & ~3u, n4 = (n + 3u) & ~3u;
     if ((size_t)(m + 128) * k4 * 4 < (1ull << 31) && ((size_t)k4 * n4 + 256) * 4 < (1ull << 31)) {
-      // where the copies fit the allocation-free entry's scratch, what is sliced fits
-      // beside them
-      const uint64_t limit = kNoallocFloats;
-      const uint64_t copies = (uint64_t)m * k4 + (uint64_t)k4 * n4;
-      const uint64_t beside =
-          copies + 64 <= limit ? std::min(max_partial_floats, limit - copies - 64) : max_partial_floats;
-      SgemmSchedule r = schedule_products(true, (int)k4, (int)n4, m, n, k4, beside);
-      const double bytes = 4.0 * ((double)m * k + (double)k * n + (double)m * k4 + (double)k4 * n4);
-      r.cost_us += 4.0 + bytes / 3.0e6;
+      SgemmSchedule r = schedule_products(true, (int)k4, (int)n4, m, n, k4, max_partial_floats);
       r.repack = true;
       r.k4 = k4;
       r.n4 = n4;
+      // where the copies fit the allocation-free entry's scratch, what is sliced fits
+      // beside them if that costs kFitsWithin at most, or 5 % where a tail's slices do not
+      // (4498x5095x1743 unsplit: 2.9 %, 2406x8816x1432 3.6 %; but 3412x1168x3645, 4 MiB
+      // past the array, 18 %)
+      const uint64_t copies = schedule_repack_floats(r, m);
+      if (schedule_scratch_floats(r, m, n) > kNoallocFloats && copies + 64 <= kNoallocFloats) {
+        SgemmSchedule fits = schedule_products(true, (int)k4, (int)n4, m, n, k4,
+                                               std::min(max_partial_floats, kNoallocFloats - copies - 64));
+        fits.repack = true;
+        fits.k4 = k4;
+        fits.n4 = n4;
+        if (fits.cost_us <= (r.tail_split ? 1.05 : kFitsWithin) * r.cost_us) r = fits;
+      }
+      const double bytes = 4.0 * ((double)m * k + (double)k * n + (double)m * k4 + (double)k4 * n4);
+      r.cost_us += 4.0 + bytes / 3.0e6;
       // slices that it cannot hold give way to copies that it can
       const bool only_copies_fit =
-          schedule_scratch_floats(s, m, n) > limit && schedule_scratch_floats(r, m, n) <= limit;
+          schedule_scratch_floats(s, m, n) > kNoallocFloats && schedule_scratch_floats(r, m, n) <= kNoallocFloats;
       if (r.cost_us < s.cost_us || only_copies_fit) s = r;
     }
   }
