@@ -848,7 +848,8 @@ PROM_REACTOR_API int prometheus_reactor_runtime_reduction_device(void* handle, c
     set_status(out_stage, out_detail_code, PROM_STAGE_INIT, PROM_REDUCTION_DETAIL_RUNTIME_UNAVAILABLE);
     return PROM_ERROR;
   }
-  std::lock_guard<std::mutex> lock(ctx().mu);  // the parts of split rows are runtime-owned
+  std::unique_lock<std::mutex> lock(ctx().mu, std::defer_lock);
+  if (row_parts_allocate(width)) lock.lock();
   if (launch_row_reduction(input, output, rows, width, operation, ctx().stream) != hipSuccess) {
     set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_REDUCTION_DETAIL_COMMAND_RECORD_FAILED);
     return PROM_ERROR;
@@ -1002,7 +1003,8 @@ PROM_REACTOR_API int prometheus_reactor_runtime_rmsnorm_device(void* handle, con
     set_status(out_stage, out_detail_code, PROM_STAGE_INIT, rt->init_detail);
     return PROM_ERROR;
   }
-  std::lock_guard<std::mutex> lock(ctx().mu);  // the parts of split rows are runtime-owned
+  std::unique_lock<std::mutex> lock(ctx().mu, std::defer_lock);
+  if (row_parts_allocate(width)) lock.lock();
   if (launch_rmsnorm(input, weight, output, inv_rms, tokens, width, input_row_stride, epsilon, ctx().stream) !=
       hipSuccess) {
     set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_DETAIL_HIP_LAUNCH_FAILED);

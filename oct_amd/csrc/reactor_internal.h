@@ -103,6 +103,7 @@ struct DeviceContext {
   hipEvent_t op_begin = nullptr, op_end = nullptr;
   void* staging[kStagingSlots] = {};
   size_t staging_bytes[kStagingSlots] = {};
+  bool row_parts = false;  // staging slot 10 was had with the device
   uint64_t staging_allocations = 0;  // hipMalloc calls made by staging(), for the diagnostics
   void* fft_roots = nullptr;  // twiddle table in staging slot 7 for length fft_roots_n
   uint32_t fft_roots_n = 0;
@@ -283,7 +284,10 @@ hipError_t launch_fft64(const double2* in, double2* out, double2* temp, const do
 // Device twiddle table for length n (cached; caller holds ctx().mu): the n/2
 // roots, followed for n > 4096 by the four-step passes' compact tables.
 const double2* fft64_roots(uint32_t n);
-// Row reductions and RMSNorm; the caller holds ctx().mu (staging slot 10).
+// Row reductions and RMSNorm.  A caller need not hold ctx().mu, which a host-pointer
+// call keeps over its copies, unless row_parts_allocate says that rows this wide may
+// have to allocate staging slot 10.
+bool row_parts_allocate(uint32_t width);
 hipError_t launch_row_reduction(const float* in, float* out, uint32_t rows, uint32_t width, uint32_t op,
                                 hipStream_t stream);
 // Binary64 reference of the same row reduction (the benchmark's correctness check).

@@ -64,7 +64,7 @@ bool ensure_device() {
   // Device address of the allocation-free SGEMM's scratch array; on failure
   // only that entry reports PROM_DETAIL_SCRATCH_UNAVAILABLE.
   (void)init_sgemm_scratch(dev);
-  (void)staging(10, kRowPartsBytes);
+  c.row_parts = staging(10, kRowPartsBytes) != nullptr;
   return true;
 }
 

@@ -26,6 +26,7 @@
 // Cross-lane steps are wave64 shuffles, cross-wave steps go through LDS; sums
 // accumulate in binary64 (free on a bandwidth-bound kernel and closest to the oracle).
 #include <algorithm>
+#include <mutex>
 
 #include "reactor_internal.h"
 
@@ -322,6 +323,14 @@ struct RowPlan {
   int waves, chunks;  // waves 0: rows over several workgroups
 };
 
+// Split rows' parts are in one buffer: one call queues its launches at a time.  Taken
+// after ctx().mu where a caller holds both.
+std::mutex g_parts_mu;
+
+size_t parts_bytes(uint32_t width) {
+  return ((size_t)width + kPartValues - 1) / kPartValues * sizeof(RowPart);
+}
+
 RowPlan plan_rows(uint32_t op, uint32_t rows, uint32_t width) {
   if (width > 32768u || (width > kPartValues && rows <= 32u)) return {0, 0};
   if (width <= 1024u) return {1, width <= 256u ? 1 : 4};
@@ -334,11 +343,12 @@ template <uint32_t kOp, bool kTail>
 hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, float* aux, uint32_t rows,
                        uint32_t width, uint32_t stride, float eps, hipStream_t stream) {
   if (p.waves == 0) {
-    const uint32_t n = (width + kPartValues - 1) / kPartValues;
+    const uint32_t n = (uint32_t)(parts_bytes(width) / sizeof(RowPart));
     // The parts' buffer is had with the device; more rows than it holds the parts of go
     // in blocks, one after the other on the stream (2^17 parts are 2^30 values).
     const uint32_t block = std::max(1u, (uint32_t)(kRowPartsBytes / sizeof(RowPart)) / n);
-    RowPart* parts = static_cast<RowPart*>(staging(10, std::max(kRowPartsBytes, (size_t)n * sizeof(RowPart))));
+    std::lock_guard<std::mutex> lock(g_parts_mu);
+    RowPart* parts = static_cast<RowPart*>(staging(10, std::max(kRowPartsBytes, parts_bytes(width))));
     if (parts == nullptr) return hipErrorOutOfMemory;
     constexpr bool kScalar = kOp == kOpSum || kOp == kOpMax;
     for (uint32_t r = 0; r < rows; r += std::min(block, rows - r)) {
@@ -429,6 +439,8 @@ __global__ __launch_bounds__(256) void row_reduction_check_kernel(const float* _
 }
 
 }  // namespace
+
+bool row_parts_allocate(uint32_t width) { return !ctx().row_parts || parts_bytes(width) > kRowPartsBytes; }
 
 hipError_t launch_row_reduction_check(const float* in, float* out, uint32_t rows, uint32_t width, uint32_t op,
                                       hipStream_t stream) {

@@ -5,6 +5,9 @@ any 4-byte address, infinities and NaN.
 Sums and the oracle accumulate in binary64, so an output carries a few fp32
 roundings of its own (exp, reciprocal, products): 8 ulps covers them.
 """
+import threading
+import time
+
 import numpy as np
 import pytest
 
@@ -133,3 +136,48 @@ def test_more_parts_than_the_buffer_holds(gpu_runtime, op):
             want, got, ulps = e / e.sum(), d.get(dst + 4 * row * width, (width,)), 8 + 2 * np.abs(v - v.max())
         assert np.all(np.abs(got - want) <= ulps * 2.0 ** -24 * np.abs(want) + 1e-37), row
     d.free()
+
+
+@pytest.mark.parametrize("op,rows,width", [(p.OP_SUM, 64, 4096), ("rmsnorm", 64, 2048), (p.OP_SOFTMAX, 8, 65536)])
+def test_device_reductions_do_not_wait_for_a_host_call(gpu_runtime, op, rows, width):
+    """A device-pointer reduction is queued at once while another thread's host-pointer
+    product (6 ms, its copies included) holds the runtime's buffers."""
+    rt = gpu_runtime
+    n = 4096
+    a = np.ones((n, n), np.float32)
+    x, w = rt.upload_new(np.ones((rows, width), np.float32)), rt.upload_new(np.ones(width, np.float32))
+    out = rt.alloc(rows * width * 4)
+
+    def reduce():
+        if op == "rmsnorm":
+            rt.rmsnorm_device(x, w, out, None, rows, width, width, 1e-6)
+        else:
+            rt.reduction_device(x, out, rows, width, op)
+
+    windows = []
+
+    def products():
+        for _ in range(3):
+            t0 = time.perf_counter()
+            rt.sgemm(n, n, n, a, a)
+            windows.append((t0, time.perf_counter()))
+
+    try:
+        reduce()
+        rt.sgemm(n, n, n, a, a)
+        thread = threading.Thread(target=products)
+        thread.start()
+        calls = []
+        while thread.is_alive() and len(calls) < 3000:
+            t0 = time.perf_counter()
+            reduce()
+            calls.append((t0, time.perf_counter()))
+            time.sleep(2e-4)
+        thread.join()
+        rt.synchronize()
+    finally:
+        for ptr in (x, w, out):
+            rt.free(ptr)
+    inside = sum(any(t0 < c0 and c1 < t1 for t0, t1 in windows) for c0, c1 in calls)
+    # one that waits for the product returns with it: at most the first and last of each
+    assert inside >= 12, (inside, len(calls), [t1 - t0 for t0, t1 in windows])
