@@ -342,6 +342,7 @@ RowPlan plan_rows(uint32_t op, uint32_t rows, uint32_t width) {
 template <uint32_t kOp, bool kTail>
 hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, float* aux, uint32_t rows,
                        uint32_t width, uint32_t stride, float eps, hipStream_t stream) {
+  constexpr bool kScalar = kOp == kOpSum || kOp == kOpMax;
   if (p.waves == 0) {
     const uint32_t n = (uint32_t)(parts_bytes(width) / sizeof(RowPart));
     // The parts' buffer is had with the device; more rows than it holds the parts of go
@@ -350,7 +351,6 @@ hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, f
     std::lock_guard<std::mutex> lock(g_parts_mu);
     RowPart* parts = static_cast<RowPart*>(staging(10, std::max(kRowPartsBytes, parts_bytes(width))));
     if (parts == nullptr) return hipErrorOutOfMemory;
-    constexpr bool kScalar = kOp == kOpSum || kOp == kOpMax;
     for (uint32_t r = 0; r < rows; r += std::min(block, rows - r)) {
       const uint32_t count = std::min(block, rows - r);
       const float* x = in + (size_t)r * stride;
@@ -366,22 +366,33 @@ hipError_t launch_rows(RowPlan p, const float* in, const float* w, float* out, f
     }
     return hipSuccess;
   }
-#define ROWS(W, C)                                                                                                   \
-  hipLaunchKernelGGL((row_kernel<kOp, W, C, kTail>), dim3(W == 1 ? (rows + 3u) / 4u : rows),                         \
-                     dim3(W == 1 ? 256 : 64 * W), 0, stream, in, w, out, aux, rows, width, stride, eps);             \
+  // A launch has fewer than 2^32 threads: more rows go in blocks (RMSNorm of 2^24 rows of
+  // four waves each, or 2^22 of sixteen).
+  const uint32_t block = (uint32_t)((1ull << 31) / (64u * (uint32_t)p.waves));
+#define ROWS(W, C)                                                                                                \
+  hipLaunchKernelGGL((row_kernel<kOp, W, C, kTail>), dim3(W == 1 ? (count + 3u) / 4u : count),                    \
+                     dim3(W == 1 ? 256 : 64 * W), 0, stream, x, w, y, aux != nullptr ? aux + r : nullptr, count,  \
+                     width, stride, eps);                                                                         \
   break
-  switch (p.waves * 100 + p.chunks) {
-    case 101: ROWS(1, 1);
-    case 104: ROWS(1, 4);
-    case 402: ROWS(4, 2);
-    case 404: ROWS(4, 4);
-    case 408: ROWS(4, 8);
-    case 1604: ROWS(16, 4);
-    case 1608: ROWS(16, 8);
-    default: return hipErrorInvalidValue;
+  for (uint32_t r = 0; r < rows; r += std::min(block, rows - r)) {
+    const uint32_t count = std::min(block, rows - r);
+    const float* x = in + (size_t)r * stride;
+    float* y = out + (kScalar ? r : (size_t)r * width);
+    switch (p.waves * 100 + p.chunks) {
+      case 101: ROWS(1, 1);
+      case 104: ROWS(1, 4);
+      case 402: ROWS(4, 2);
+      case 404: ROWS(4, 4);
+      case 408: ROWS(4, 8);
+      case 1604: ROWS(16, 4);
+      case 1608: ROWS(16, 8);
+      default: return hipErrorInvalidValue;
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
   }
 #undef ROWS
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 // Rows of whole 16-byte chunks at 16-byte addresses take the kernels without tails.
