@@ -1104,26 +1104,53 @@ Rows operand_rows(bool aligned, int lda, long long sa, int ldb, long long sb, ui
   return staged_buffer_path(lda, ldb, m, n, k) ? Rows::kUnaligned : Rows::kScalar;
 }
 
-double plan_cost(const SgemmPlan& p, uint32_t m, uint32_t n, uint32_t batch, Rows rows = Rows::kAligned) {
-  const int t = p.tile;
-  const double w_total = (double)((m + kTileM[t] - 1) / kTileM[t]) * ((n + kTileN[t] - 1) / kTileN[t]) * p.splits *
-                         batch;
+// us per K step of 16 of each workgroup, with w + 1 of them resident per CU.
+struct TileSteps {
+  double us[kTileShapes][5];
+};
+
+constexpr TileSteps tile_steps() {
+  TileSteps s{};
+  for (int t = 0; t < kTileShapes; ++t)
+    for (int w = 0; w < kTileOcc[t]; ++w) s.us[t][w] = kTileM[t] * kTileN[t] * 32.0 / 609280.0 / kTileEffW[t][w];
+  return s;
+}
+
+constexpr TileSteps kSteps = tile_steps();
+
+// The part of the estimate that the K slices do not change.  A plan tries up to 64
+// (tile, slices) pairs, three times where the rows leave a tail, on the host and on
+// every call, so what the tile alone decides is kept out of that loop.
+struct TileGrid {
+  int tile;
+  double workgroups;  // of one slice
+};
+
+TileGrid tile_grid(int t, uint32_t m, uint32_t n, uint32_t batch) {
+  return {t, (double)((m + kTileM[t] - 1) / kTileM[t]) * ((n + kTileN[t] - 1) / kTileN[t]) * batch};
+}
+
+double plan_cost(const TileGrid& g, const SgemmPlan& p, uint32_t m, uint32_t n, Rows rows) {
+  const int t = g.tile, occ = kTileOcc[t];
+  const double w_total = g.workgroups * p.splits;
   const double k_tiles = (double)((p.k_len + kBK - 1) / kBK);
-  const double t16 = (double)kTileM[t] * kTileN[t] * 32.0 / 609280.0;
-  const double slots = 256.0 * kTileOcc[t];
-  const double full = std::floor(w_total / slots);
+  const double slots = 256.0 * occ;
+  const double full = w_total < slots ? 0.0 : std::floor(w_total / slots);
   const double rest = w_total - full * slots;
-  auto eff = [&](int w) { return kTileEffW[t][std::min(w, kTileOcc[t]) - 1]; };
-  double us = full * kTileOcc[t] * k_tiles * t16 / eff(kTileOcc[t]);
+  double us = full * occ * k_tiles * kSteps.us[t][occ - 1];
   if (rest > 0) {
-    const int w = (int)std::ceil(rest / 256.0);
-    us += w * k_tiles * t16 / eff(w);
+    const int w = (int)std::ceil(rest * (1.0 / 256.0));
+    us += w * k_tiles * kSteps.us[t][w - 1];
   }
   if (t < 3 && rows == Rows::kUnaligned) us = 1.15 * us + 1.3;
   if (t < 3 && rows == Rows::kScalar) us *= 1.5;
   us += 3.45 + 1.72 * (full + (rest > 0 ? 1.0 : 0.0));
-  if (p.splits > 1) us += 1.46 + (double)(p.splits + 1) * m * n * 4.0 / 3.5e6;
+  if (p.splits > 1) us += 1.46 + (double)(p.splits + 1) * m * n * (4.0 / 3.5e6);
   return us;
+}
+
+double plan_cost(const SgemmPlan& p, uint32_t m, uint32_t n, uint32_t batch, Rows rows = Rows::kAligned) {
+  return plan_cost(tile_grid(p.tile, m, n, batch), p, m, n, rows);
 }
 
 // max_partial_floats bounds the split-K partial buffer (splits * m * n floats)
@@ -1136,25 +1163,31 @@ SgemmPlan plan_sgemm(bool aligned, int lda, long long sa, int ldb, long long sb,
   // model is accurate to a few per cent).
   static const int kTileOrder[kTileShapes + 1] = {4, 3, 0, 1, 2, 5, 6, 7, 4};
   const Rows kind = operand_rows(aligned, lda, sa, ldb, sb, m, n, k);
+  const bool direct = buffer_path(aligned, lda, sa, ldb, sb, m, n, k);
+  const uint64_t slab = (uint64_t)m * n;
+  // a slice has 64 k at least
+  const int most_splits = batch > 1 ? 1 : (int)std::max(1u, std::min(16u, k / 64u));
   SgemmPlan best = make_plan(0, 1, k);
   double best_cost = 1e300;
   for (int i = 0; i <= kTileShapes; ++i) {
     const int t = kTileOrder[i];
     const bool last = i == kTileShapes;
+    if (t >= 3 && !direct) continue;
+    // K tails: the 64x64 tiles, and 128x128, whose offsets (to a K tile past B) stay
+    // below 2^32 if B has a K tile itself.  Unsliced, as slices of tall products would
+    // need more scratch than the allocation-free entry has, and as the last
+    // candidate, so that among the others the choice is as without it.
     if (last && k % kBK == 0) break;
+    if (k % kBK != 0 && (t == 3 || t == 7 || (t == 4 && (!last || k < (uint32_t)kBK)))) continue;
+    // (sliced, 64x128 measured within 2 % of the other tiles)
+    const int most = t == 7 || last ? 1 : most_splits;
+    const TileGrid grid = tile_grid(t, m, n, batch);
     for (int s : kSplitChoices) {
-      if (s > 1 && (batch > 1 || k / (uint32_t)s < 64)) break;
-      if (s > 1 && t == 7) break;  // sliced, 64x128 measured within 2 % of the other tiles
+      if (s > most) break;
       const SgemmPlan p = make_plan(t, s, k);
       if (p.splits != s) continue;
-      if (p.splits > 1 && (uint64_t)p.splits * m * n > max_partial_floats) continue;
-      if (t >= 3 && !buffer_path(aligned, lda, sa, ldb, sb, m, n, k)) continue;
-      // K tails: the 64x64 tiles, and 128x128, whose offsets (to a K tile past B) stay
-      // below 2^32 if B has a K tile itself.  Unsliced, as slices of tall products would
-      // need more scratch than the allocation-free entry has, and as the last
-      // candidate, so that among the others the choice is as without it.
-      if (k % kBK != 0 && (t == 3 || t == 7 || (t == 4 && (s > 1 || !last || k < (uint32_t)kBK)))) continue;
-      const double c = plan_cost(p, m, n, batch, kind);
+      if (s > 1 && (uint64_t)s * slab > max_partial_floats) break;
+      const double c = plan_cost(grid, p, m, n, kind);
       if (c < best_cost * 0.99) {
         best_cost = c;
         best = p;

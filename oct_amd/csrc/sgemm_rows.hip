@@ -69,7 +69,8 @@ double rows_us(const RowsShape& q, int splits, uint32_t m, uint32_t n, uint32_t 
   const double load = (double)(groups / 256) + (rest > 0 ? kPartCu + (1.0 - kPartCu) * rest / 256.0 : 0.0);
   const double run = std::max(load * slice * step, std::ceil((double)slice / q.w) * q.chain);
   const double read = (double)k * n * halves * 4.0 / kReadBytesPerUs;
-  double us = kLaunchUs + std::pow(std::pow(run, 4.0) + std::pow(read, 4.0), 0.25);
+  const double run2 = run * run, read2 = read * read;
+  double us = kLaunchUs + std::sqrt(std::sqrt(run2 * run2 + read2 * read2));
   if (splits > 1) us += kReduceUs + (double)(splits + 1) * m * n * 4.0 / kReduceBytesPerUs;
   return us;
 }

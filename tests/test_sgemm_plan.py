@@ -6,6 +6,7 @@ up here first."""
 from __future__ import annotations
 
 import ctypes
+import time
 
 import pytest
 
@@ -187,3 +188,20 @@ def test_copies_past_the_noalloc_scratch_keep_their_slices(m, n, k, most_us):
     rc, i = _plan(m, n, k)
     assert rc == p.PROM_OK and i.repacked == 1 and max(i.k_slices[:i.products]) > 1
     assert i.estimated_us <= most_us
+
+
+def test_planning_few_rows_takes_little_longer_than_planning_tiles():
+    """The plan is made on the host in every call, so for the smallest products it counts as
+    the kernel does (15x2048x1536: 6.6 us of planning beside a call of 7.2 before the pairs'
+    shared terms left the loop, 2.4 after).  Compared with a plan of tiles alone, 2.3 times
+    as long then, 1.3 to 1.4 now."""
+    lib, info = p.shared_library(), p.PrometheusSgemmPlanInfo()
+    info.struct_size = ctypes.sizeof(info)
+    best = {}
+    for _ in range(30):
+        for shape in ((15, 2048, 1536), (1024, 1024, 1024)):
+            t0 = time.perf_counter()
+            for _ in range(200):
+                lib.prometheus_reactor_sgemm_plan(*shape, ctypes.byref(info))
+            best[shape] = min(best.get(shape, 1.0), time.perf_counter() - t0)
+    assert best[15, 2048, 1536] < 1.8 * best[1024, 1024, 1024], best
