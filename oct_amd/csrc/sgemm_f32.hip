@@ -205,11 +205,17 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
     }
   };
 
-  floatx16 acc[T::kMI][T::kNI];
+  // Two sums per output, of every other k step (one for 128x256, whose 256 registers of sums
+  // would not fit): half the roundings in a chain, as in the 64x64 tiles that otherwise run
+  // unaligned operands on padded copies.
+  constexpr int kSums = kBM * kBN <= 128 * 128 ? 2 : 1;
+  floatx16 acc[kSums][T::kMI][T::kNI];
 #pragma unroll
-  for (int i = 0; i < T::kMI; ++i)
+  for (int q = 0; q < kSums; ++q)
 #pragma unroll
-    for (int j = 0; j < T::kNI; ++j) acc[i][j] = floatx16{};
+    for (int i = 0; i < T::kMI; ++i)
+#pragma unroll
+      for (int j = 0; j < T::kNI; ++j) acc[q][i][j] = floatx16{};
 
   const int k_tiles = (K + kBK - 1) / kBK;
   load_tile(0);
@@ -244,10 +250,17 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
       for (int i = 0; i < T::kMI; ++i)
 #pragma unroll
         for (int j = 0; j < T::kNI; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a_op[s & 1][i], b_op[s & 1][j], acc[i][j], 0, 0, 0);
+          acc[s % kSums][i][j] =
+              __builtin_amdgcn_mfma_f32_32x32x2f32(a_op[s & 1][i], b_op[s & 1][j], acc[s % kSums][i][j], 0, 0, 0);
     }
     if (more) store_tile(cur ^ 1);
     __syncthreads();
+  }
+  if constexpr (kSums == 2) {
+#pragma unroll
+    for (int i = 0; i < T::kMI; ++i)
+#pragma unroll
+      for (int j = 0; j < T::kNI; ++j) acc[0][i][j] += acc[1][i][j];
   }
 
   // Accumulator layout of a 32x32 MFMA block: lane l, register r holds
@@ -271,7 +284,7 @@ __global__ __launch_bounds__(256, (kBM * kBN >= 128 * 256 ? 2 : 3)) void sgemm_f
 #pragma unroll
   for (int i = 0; i < T::kMI; ++i)
 #pragma unroll
-    for (int j = 0; j < T::kNI; ++j) store_block(acc[i][j], i, j);
+    for (int j = 0; j < T::kNI; ++j) store_block(acc[0][i][j], i, j);
 }
 
 // Direct-to-LDS variant for operands with 16-byte rows (k, lda, ldb multiples of
@@ -309,8 +322,10 @@ struct DlCfg {
 // kTail (128x128 tiles, K a multiple of 4 but not of the K tile): the last tile's B
 // rows past K read zero (outside the buffer range), and its A columns past K, which
 // the transfers fill from the next row, are cleared in LDS before that tile is used.
-// The sums are taken in two, of the first and the second half of each K tile: the
-// 64x64 tiles, the other kernels for such a K, add two as well, and 4097x3001x513 keeps their error (2.9e-7 of the
+//
+// kTwoSums: each output is the sum of two, over the first and the second half of each K
+// tile.  The 64x64 tiles, the other kernels for a K tail and for row counts that 128
+// divides badly, add two as well, and 4097x3001x513 keeps their error (2.9e-7 of the
 // result against 64 bits; 4.1e-7 in one chain) at 128x128's speed: 114 us, 124 before.
 template <int kBN, int kBM, bool kGeGLU = false, bool kTail = false>
 __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, const float* __restrict__ B, float* C,
@@ -327,6 +342,7 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
   constexpr int kABlocks = kBM / 16, kBBlocks = kBN == 256 ? 16 : 8;  // 1 KB transfers per K tile
   constexpr int kAI = kABlocks / kWaves;
   constexpr int kBI = (kBBlocks + kWaves - 1) / kWaves;
+  constexpr bool kTwoSums = kTail || (kBM == 64 && !kGeGLU);
   static_assert(kABlocks == kAI * kWaves, "whole A transfers per wave");
   typedef __attribute__((address_space(3))) void lds_void;
 
@@ -419,13 +435,13 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
   }
 
   floatx16 acc[kMI][kNI];
-  floatx16 acc_odd[kTail ? kMI : 1][kTail ? kNI : 1];  // kTail: the second half of each K tile
+  floatx16 acc_odd[kTwoSums ? kMI : 1][kTwoSums ? kNI : 1];  // kTwoSums: the second half of each K tile
 #pragma unroll
   for (int i = 0; i < kMI; ++i)
 #pragma unroll
     for (int j = 0; j < kNI; ++j) {
       acc[i][j] = floatx16{};
-      if constexpr (kTail) acc_odd[i][j] = floatx16{};
+      if constexpr (kTwoSums) acc_odd[i][j] = floatx16{};
     }
 
   auto compute = [&](const char* st) {
@@ -450,7 +466,7 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
         for (int mi = 0; mi < kMI; ++mi)
 #pragma unroll
           for (int ni = 0; ni < kNI; ++ni) {
-            floatx16& sum = kTail && p == 1 ? acc_odd[kTail ? mi : 0][kTail ? ni : 0] : acc[mi][ni];
+            floatx16& sum = kTwoSums && p == 1 ? acc_odd[kTwoSums ? mi : 0][kTwoSums ? ni : 0] : acc[mi][ni];
             sum = __builtin_amdgcn_mfma_f32_32x32x2f32(a[mi][j], b[ni], sum, 0, 0, 0);
           }
       }
@@ -494,7 +510,7 @@ __device__ __forceinline__ void sgemm_f32_dl_body(const float* __restrict__ A, c
     if constexpr (kTail) settle_last(S0);
     compute(S0);
   }
-  if constexpr (kTail) {
+  if constexpr (kTwoSums) {
 #pragma unroll
     for (int i = 0; i < kMI; ++i)
 #pragma unroll

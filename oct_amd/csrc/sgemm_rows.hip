@@ -13,7 +13,7 @@
 //     k = k0 + 4 g + c, and lane (g, j) loads kC consecutive columns of that row
 //     of B (16 kC floats of a row per group); each of them feeds one MFMA;
 //   * a workgroup owns 16 kC columns; its waves take the granules of its K slice in
-//     turn and add their sums through LDS in wave order at the end (deterministic);
+//     turn and add their sums through LDS in a fixed order at the end (deterministic);
 //   * where that leaves CUs idle K is also cut into slices over gridDim.y, whose
 //     slabs a second kernel adds in slice order.
 //
@@ -135,7 +135,7 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
           if (k0 + 4 * grp + c >= p.k) q.a[mb][c] = 0.0f;
     }
   };
-  // Sums of four granules (64 of k) at a time go into `total`: a chain of 64 and one of
+  // Sums of two granules (32 of k) at a time go into `total`: a chain of 32 and one of
   // the blocks, whose rounding is that of the tiles' K slices or less where one chain
   // over a long K has more (13x9344x7680: 5.6e-7 of the result, the tiles 3.3e-7).
   floatx4 acc[kH][kMB][kC], total[kH][kMB][kC];
@@ -178,7 +178,7 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
     Granule next;
     load(next, g + kW);
     compute(q);
-    if ((done & 3) == 0) add_up();
+    if ((done & 1) == 0) add_up();
     q = next;
   }
   if (g < g1) compute(q);
@@ -196,18 +196,22 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
         for (int i = 0; i < 4; ++i)
           sums[wave][((h * 16 * kMB) + 16 * mb + 4 * grp + i) * kCols + kC * li + j] = total[h][mb][j][i];
   __syncthreads();
+  // The waves' sums, added in pairs: log2(kW) roundings each, in a fixed order.
+  auto sum_waves = [&](int e) __attribute__((always_inline)) {
+    float v[kW];
+#pragma unroll
+    for (int w = 0; w < kW; ++w) v[w] = sums[w][e];
+#pragma unroll
+    for (int step = kW / 2; step > 0; step /= 2)
+#pragma unroll
+      for (int w = 0; w < step; ++w) v[w] += v[w + step];
+    return v[0];
+  };
   float* out = p.c + (gridDim.y > 1 ? blockIdx.y * p.slab : 0);
   for (int e = tid; e < 16 * kMB * kCols; e += 64 * kW) {
     const int i = e / kCols, col = col0 + e % kCols;
-    float v = sums[0][e];
-#pragma unroll
-    for (int w = 1; w < kW; ++w) v += sums[w][e];
-    if constexpr (kGe) {
-      float u = sums[0][e + kBlock / 2];
-#pragma unroll
-      for (int w = 1; w < kW; ++w) u += sums[w][e + kBlock / 2];
-      v = gelu_tanh(v) * u;
-    }
+    float v = sum_waves(e);
+    if constexpr (kGe) v = gelu_tanh(v) * sum_waves(e + kBlock / 2);
     if (i < p.m && col < p.n) {
       if (p.r != nullptr) v += p.r[(size_t)i * p.ldr + col];
       out[(size_t)i * p.ldc + col] = v;
