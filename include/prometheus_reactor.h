@@ -725,6 +725,35 @@ PROM_REACTOR_API int prometheus_reactor_sgemm_plan(uint32_t m, uint32_t n, uint3
 PROM_REACTOR_API int prometheus_reactor_runtime_gemm_bf16_device(void* handle, const uint16_t* a, const uint16_t* b,
                                                                  float* c, uint32_t m, uint32_t n, uint32_t k,
                                                                  uint32_t* out_stage, int* out_detail_code);
+/* No counterpart in the reference (no bf16 GEMM there): the kernel that
+   ..._gemm_bf16_device, or a product of the DiT block, runs for a shape with
+   contiguous 16-byte aligned operands, as a pure function of the shape, and one
+   product with a caller-chosen kernel, for tuning and per-kernel tests.
+   tile: 0 = 32x128, 1 = 64x64, 2 = 64x128, 3 = 64x256, 4 = 128x128, 5 =
+   192x128, 6 = 128x256, 7 = 192x256, 8 = 256x256 (K tiles of 64), 9 = 256x256
+   with K tiles of 32 in five stages, 10 = 128x128 staged through registers;
+   k_slices 1..16, more than 1 for tiles 0-8 only (the sums of the slices are
+   added by a second launch).  flags: PROM_GEMM_BF16_SWIGLU: b is [k, 2n] =
+   [gate | up] and the output bf16 [m, n], silu(a @ gate) * (a @ up) (tiles 2-4,
+   6-9, one slice); PROM_GEMM_BF16_BLOCKED_A (plan only): a can be stored K-blocked, as
+   the DiT block's row kernels store it for tile 9.  The plan's out_padded says
+   that operands are first copied to zero-padded buffers.  Without a fused
+   kernel for a SwiGLU shape, or for a shape that is not admitted, the plan
+   returns PROM_ERROR.  A variant that cannot run the shape or the operands'
+   alignment (tiles 0-8: k, and b's columns, multiples of 8; 9: k a multiple of
+   32, n of 8, with SwiGLU of 128; 16-byte aligned operands) returns
+   PROM_ERROR, stage INIT, PROM_DETAIL_INVALID_ARGUMENT; otherwise the device
+   entry's statuses. */
+#define PROM_GEMM_BF16_SWIGLU 1u
+#define PROM_GEMM_BF16_BLOCKED_A 2u
+PROM_REACTOR_API int prometheus_reactor_gemm_bf16_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t flags,
+                                                       uint32_t* out_tile, uint32_t* out_k_slices,
+                                                       uint32_t* out_padded);
+PROM_REACTOR_API int prometheus_reactor_runtime_gemm_bf16_device_variant(void* handle, const uint16_t* a,
+                                                                         const uint16_t* b, void* c, uint32_t m,
+                                                                         uint32_t n, uint32_t k, uint32_t tile,
+                                                                         uint32_t k_slices, uint32_t flags,
+                                                                         uint32_t* out_stage, int* out_detail_code);
 /* operation as PrometheusReductionRequest; softmax writes rows*width, sum/max rows. */
 PROM_REACTOR_API int prometheus_reactor_runtime_reduction_device(void* handle, const float* input, float* output,
                                                                  uint32_t rows, uint32_t width, uint32_t operation,

@@ -598,6 +598,12 @@ namespace {
 
 enum class Bf16Path { kFiveStage, kTiles, kPadded, kSmall };
 
+// The five-stage kernel takes whole K tiles and byte offsets below 2^31 (of operands that
+// bf16_tiles_take accepts).
+bool five_stage_range(int lda, int ldb, uint32_t m, uint32_t k) {
+  return k % kBK4 == 0 && (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * ldb * 2 < (1ull << 31);
+}
+
 // The kernel launch_gemm_bf16_ex runs for a shape and its operands' layout: the
 // least estimate of the 256x256 five-stage kernel (whole K tiles of 32 only) and
 // the tiles of gemm_bf16_tiles.hip.  `blocked`: A is or can be stored K-blocked, which
@@ -610,9 +616,8 @@ Bf16Path bf16_path(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint3
                    Bf16TilePlan* plan, bool blocked) {
   *plan = plan_bf16_tiles(m, n, k, false);
   if (bf16_tiles_take(a, lda, b, ldb, k)) {
-    const bool range = (size_t)(m + kBM2) * lda * 2 < (1ull << 31) && (size_t)k * ldb * 2 < (1ull << 31);
     const double five_us = bf16_five_stage_us(m, n, k, 0) * (blocked ? 0.965 : 1.0);
-    return range && k % kBK4 == 0 && five_us < plan->us ? Bf16Path::kFiveStage : Bf16Path::kTiles;
+    return five_stage_range(lda, ldb, m, k) && five_us < plan->us ? Bf16Path::kFiveStage : Bf16Path::kTiles;
   }
   if (k >= (1u << 22) - 8 || n >= (1u << 23) - 8) return Bf16Path::kSmall;
   const double tiles128 = (double)((m + kBM - 1) / kBM) * ((n + kBN - 1) / kBN);
@@ -654,6 +659,43 @@ bool blocked_range(int a_slice, uint32_t m, uint32_t k) {
   return a_slice >= (int)((m + kBM2 - 1) / kBM2 * kBM2) && (size_t)k * a_slice * 2 < (1ull << 31);
 }
 
+// The SwiGLU form of the 256x256 five-stage kernel, whole tiles only.
+hipError_t launch_swiglu_five_stage(const uint16_t* a, int lda, const uint16_t* w13, uint16_t* h, int ldh, uint32_t m,
+                                    uint32_t f, uint32_t k, hipStream_t stream, int a_slice, int h_slice) {
+  const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
+  const int tiles_n2 = (int)(f / 128);
+  const int total = tiles_m2 * tiles_n2;
+  hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, dim3((unsigned)total), dim3(512), 0, stream, a, w13, (int)m, (int)f,
+                     (int)k, tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, total, 1, nullptr, a_slice, h_slice);
+  return hipGetLastError();
+}
+
+// The 256x256 five-stage kernel and the register-staged 128x128 kernel.
+hipError_t launch_five_stage(const uint16_t* a, int lda, const uint16_t* b, int ldb, float* c, uint16_t* cb, int ldc,
+                             uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr, hipStream_t stream,
+                             int a_slice) {
+  const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
+  const int tiles_n2 = (int)((n + kBN2 - 1) / kBN2);
+  hipLaunchKernelGGL(gemm_bf16_dl4_kernel, dim3((unsigned)(tiles_m2 * tiles_n2)), dim3(512), 0, stream, a, b, c,
+                     (int)m, (int)n, (int)k, tiles_m2, tiles_n2, lda, ldb, ldc, residual, ldr, cb, a_slice);
+  return hipGetLastError();
+}
+
+hipError_t launch_staged(const uint16_t* a, int lda, const uint16_t* b, int ldb, float* c, uint16_t* cb, int ldc,
+                         uint32_t m, uint32_t n, uint32_t k, const float* residual, int ldr, hipStream_t stream) {
+  const int tiles_m = (int)((m + kBM - 1) / kBM);
+  const int tiles_n = (int)((n + kBN - 1) / kBN);
+  const dim3 grid((unsigned)(tiles_m * tiles_n));
+  const bool vec = k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned16(a) && aligned16(b);
+  if (vec)
+    hipLaunchKernelGGL(gemm_bf16_mfma_kernel<true>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
+                       tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
+  else
+    hipLaunchKernelGGL(gemm_bf16_mfma_kernel<false>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
+                       tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
+  return hipGetLastError();
+}
+
 }  // namespace
 
 bool gemm_bf16_takes_blocked_a(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t m, uint32_t n,
@@ -674,13 +716,8 @@ hipError_t launch_gemm_bf16_ex(const uint16_t* a, int lda, const uint16_t* b, in
   Bf16Path path = bf16_path(a, lda, b, ldb, m, n, k, &plan, a_slice > 0);
   if (a_slice > 0 && (path != Bf16Path::kFiveStage || !blocked_range(a_slice, m, k))) return hipErrorNotSupported;
   if (path_detail) *path_detail = PROM_DETAIL_PATH_HIP_MFMA_BF16;
-  if (path == Bf16Path::kFiveStage) {
-    const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
-    const int tiles_n2 = (int)((n + kBN2 - 1) / kBN2);
-    hipLaunchKernelGGL(gemm_bf16_dl4_kernel, dim3((unsigned)(tiles_m2 * tiles_n2)), dim3(512), 0, stream, a, b, c,
-                       (int)m, (int)n, (int)k, tiles_m2, tiles_n2, lda, ldb, ldc, residual, ldr, cb, a_slice);
-    return hipGetLastError();
-  }
+  if (path == Bf16Path::kFiveStage)
+    return launch_five_stage(a, lda, b, ldb, c, cb, ldc, m, n, k, residual, ldr, stream, a_slice);
   if (path == Bf16Path::kPadded) {
     const bool copy_a = k % 8 != 0 || lda % 8 != 0 || !aligned16(a);
     const bool copy_b = ldb % 8 != 0 || !aligned16(b);
@@ -706,17 +743,7 @@ hipError_t launch_gemm_bf16_ex(const uint16_t* a, int lda, const uint16_t* b, in
   }
   if (path != Bf16Path::kSmall)
     return launch_bf16_tiles(plan, false, a, lda, b, ldb, c, cb, ldc, m, n, k, residual, ldr, stream);
-  const int tiles_m = (int)((m + kBM - 1) / kBM);
-  const int tiles_n = (int)((n + kBN - 1) / kBN);
-  const dim3 grid((unsigned)(tiles_m * tiles_n));
-  const bool vec = k % 8 == 0 && n % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && aligned16(a) && aligned16(b);
-  if (vec)
-    hipLaunchKernelGGL(gemm_bf16_mfma_kernel<true>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
-                       tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
-  else
-    hipLaunchKernelGGL(gemm_bf16_mfma_kernel<false>, grid, dim3(256), 0, stream, a, b, c, (int)m, (int)n, (int)k,
-                       tiles_m, tiles_n, lda, ldb, ldc, residual, ldr, cb);
-  return hipGetLastError();
+  return launch_staged(a, lda, b, ldb, c, cb, ldc, m, n, k, residual, ldr, stream);
 }
 
 hipError_t launch_gemm_bf16_swiglu(const uint16_t* a, int lda, const uint16_t* w13, uint16_t* h, int ldh, uint32_t m,
@@ -733,7 +760,6 @@ hipError_t launch_gemm_bf16_swiglu(const uint16_t* a, int lda, const uint16_t* w
   }
   const int tiles_m2 = (int)((m + kBM2 - 1) / kBM2);
   const int tiles_n2 = (int)(f / 128);
-  const dim3 grid((unsigned)(tiles_m2 * tiles_n2));
   // K-blocked A or H.
   if ((a_slice > 0 && !blocked_range(a_slice, m, k)) ||
       (h_slice > 0 && (h_slice < tiles_m2 * kBM2 || (size_t)f * h_slice * 2 >= (1ull << 31))))
@@ -757,11 +783,60 @@ hipError_t launch_gemm_bf16_swiglu(const uint16_t* a, int lda, const uint16_t* w
                        reinterpret_cast<const float2*>(part_ws), h, ldh, (int)m, tiles_m2, tiles_n2, n_main, splits,
                        h_slice);
     if (launches) *launches = 2;
-  } else {
-    hipLaunchKernelGGL(gemm_bf16_dl4_swiglu_kernel, grid, dim3(512), 0, stream, a, w13, (int)m, (int)f, (int)k,
-                       tiles_m2, tiles_n2, lda, (int)(2 * f), ldh, h, total, 1, nullptr, a_slice, h_slice);
+    return hipGetLastError();
   }
-  return hipGetLastError();
+  return launch_swiglu_five_stage(a, lda, w13, h, ldh, m, f, k, stream, a_slice, h_slice);
+}
+
+bool plan_gemm_bf16(uint32_t m, uint32_t n, uint32_t k, bool swiglu, bool blocked_a, uint32_t* tile, uint32_t* slices,
+                    bool* padded) {
+  Bf16TilePlan plan;
+  *padded = false;
+  *slices = 1;
+  if (swiglu) {
+    if (swiglu_five_stage(nullptr, (int)k, nullptr, m, n, k)) {
+      *tile = kBf16FiveStage;
+      return true;
+    }
+    if (!swiglu_tiles_ok(nullptr, (int)k, nullptr, n, k)) return false;
+    plan = plan_bf16_tiles(m, 2 * n, k, true);
+  } else {
+    const Bf16Path path = bf16_path(nullptr, (int)k, nullptr, (int)n, m, n, k, &plan, blocked_a);
+    if (path == Bf16Path::kFiveStage || path == Bf16Path::kSmall) {
+      *tile = path == Bf16Path::kFiveStage ? kBf16FiveStage : kBf16Staged;
+      return true;
+    }
+    *padded = path == Bf16Path::kPadded;
+  }
+  *tile = (uint32_t)plan.tile;
+  *slices = (uint32_t)plan.splits;
+  return true;
+}
+
+hipError_t launch_gemm_bf16_variant(const uint16_t* a, const uint16_t* b, void* c, uint32_t m, uint32_t n, uint32_t k,
+                                    uint32_t tile, uint32_t slices, bool swiglu, hipStream_t stream) {
+  float* cf = static_cast<float*>(c);
+  uint16_t* cb = static_cast<uint16_t*>(c);
+  const int ldb = (int)(swiglu ? 2 * n : n);
+  if (slices < 1 || slices > 16) return hipErrorInvalidValue;
+  if (tile < kBf16FiveStage) {
+    if (!bf16_tiles_take(a, (int)k, b, ldb, k) || (k + 63) / 64 < slices) return hipErrorInvalidValue;
+    if (swiglu && (slices > 1 || n % 8 != 0 || !bf16_tile_has_swiglu(tile))) return hipErrorInvalidValue;
+    return launch_bf16_tiles(Bf16TilePlan{(int)tile, (int)slices, 0.0}, swiglu, a, (int)k, b, ldb,
+                             swiglu ? nullptr : cf, swiglu ? cb : nullptr, (int)n, m, n, k, nullptr, 0, stream);
+  }
+  if (slices != 1) return hipErrorInvalidValue;
+  if (tile == kBf16FiveStage && swiglu)
+    return swiglu_five_stage_ok(a, (int)k, b, m, n, k)
+               ? launch_swiglu_five_stage(a, (int)k, b, cb, (int)n, m, n, k, stream, 0, 0)
+               : hipErrorInvalidValue;
+  if (tile == kBf16FiveStage)
+    return bf16_tiles_take(a, (int)k, b, ldb, k) && five_stage_range((int)k, ldb, m, k)
+               ? launch_five_stage(a, (int)k, b, ldb, cf, nullptr, (int)n, m, n, k, nullptr, 0, stream, 0)
+               : hipErrorInvalidValue;
+  if (tile == kBf16Staged && !swiglu)
+    return launch_staged(a, (int)k, b, ldb, cf, nullptr, (int)n, m, n, k, nullptr, 0, stream);
+  return hipErrorInvalidValue;
 }
 
 hipError_t launch_gemm_bf16(const uint16_t* a, const uint16_t* b, float* c, uint32_t m, uint32_t n, uint32_t k,

@@ -544,6 +544,10 @@ Bf16TilePlan plan_bf16_tiles(uint32_t m, uint32_t n, uint32_t k, bool swiglu) {
   return best;
 }
 
+static_assert(kNumTiles == (int)kBf16FiveStage, "the kernels' numbers");
+
+bool bf16_tile_has_swiglu(uint32_t tile) { return tile < (uint32_t)kNumTiles && kTiles[tile].ni == 2; }
+
 bool bf16_tiles_take(const uint16_t* a, int lda, const uint16_t* b, int ldb, uint32_t k) {
   return k % 8 == 0 && lda % 8 == 0 && ldb % 8 == 0 && ((uintptr_t)a & 15u) == 0 && ((uintptr_t)b & 15u) == 0 &&
          tiles_in_range(lda, ldb);

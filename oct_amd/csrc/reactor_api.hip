@@ -691,6 +691,48 @@ PROM_REACTOR_API int prometheus_reactor_runtime_gemm_bf16_device(void* handle, c
   return gemm_device<uint16_t>(handle, a, b, c, m, n, k, out_stage, out_detail_code, launch_gemm_bf16);
 }
 
+PROM_REACTOR_API int prometheus_reactor_gemm_bf16_plan(uint32_t m, uint32_t n, uint32_t k, uint32_t flags,
+                                                       uint32_t* out_tile, uint32_t* out_k_slices,
+                                                       uint32_t* out_padded) {
+  if (out_tile == nullptr || out_k_slices == nullptr || out_padded == nullptr) return PROM_ERROR;
+  *out_tile = *out_k_slices = *out_padded = 0;
+  const bool swiglu = (flags & PROM_GEMM_BF16_SWIGLU) != 0u;
+  if (m == 0u || n == 0u || k == 0u || (swiglu && n > 0x3fffffffu) || !gemm_shape_fits(m, swiglu ? 2 * n : n, k))
+    return PROM_ERROR;
+  bool padded = false;
+  if (!plan_gemm_bf16(m, n, k, swiglu, (flags & PROM_GEMM_BF16_BLOCKED_A) != 0u, out_tile, out_k_slices, &padded))
+    return PROM_ERROR;
+  *out_padded = padded;
+  return PROM_OK;
+}
+
+// As ..._sgemm_device_variant, for the bf16 kernels (no reference counterpart).
+PROM_REACTOR_API int prometheus_reactor_runtime_gemm_bf16_device_variant(void* handle, const uint16_t* a,
+                                                                         const uint16_t* b, void* c, uint32_t m,
+                                                                         uint32_t n, uint32_t k, uint32_t tile,
+                                                                         uint32_t k_slices, uint32_t flags,
+                                                                         uint32_t* out_stage, int* out_detail_code) {
+  Runtime* rt = lookup(handle);
+  const bool swiglu = (flags & PROM_GEMM_BF16_SWIGLU) != 0u;
+  const int v = gemm_validate(rt, a, b, c, m, swiglu && n <= 0x3fffffffu ? 2 * n : n, k, out_stage, out_detail_code);
+  if (v != PROM_OK) return v;
+  DeviceContext& cx = ctx();
+  std::lock_guard<std::mutex> lock(cx.mu);
+  const hipError_t e = swiglu && n > 0x3fffffffu
+                           ? hipErrorInvalidValue
+                           : launch_gemm_bf16_variant(a, b, c, m, n, k, tile, k_slices, swiglu, cx.stream);
+  if (e == hipErrorInvalidValue) {
+    set_status(out_stage, out_detail_code, PROM_STAGE_INIT, PROM_DETAIL_INVALID_ARGUMENT);
+    return PROM_ERROR;
+  }
+  if (e != hipSuccess) {
+    set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_DETAIL_HIP_LAUNCH_FAILED);
+    return PROM_ERROR;
+  }
+  set_status(out_stage, out_detail_code, PROM_STAGE_SUBMIT, PROM_DETAIL_PATH_HIP_MFMA_BF16);
+  return PROM_OK;
+}
+
 PROM_REACTOR_API int prometheus_reactor_reduction_plan(const PrometheusReductionRequest* request,
                                                         PrometheusReductionPlan* out_plan) {
   if (out_plan == nullptr) return PROM_ERROR;

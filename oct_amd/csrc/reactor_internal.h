@@ -261,6 +261,16 @@ hipError_t launch_bf16_tiles(Bf16TilePlan plan, bool swiglu, const uint16_t* a, 
                              const float* residual, int ldr, hipStream_t stream);
 hipError_t launch_bf16_pad_rows(const uint16_t* src, uint16_t* dst, uint32_t rows, uint32_t cols, int ld_s, int ld_d,
                                 hipStream_t stream);
+constexpr uint32_t kBf16FiveStage = 9, kBf16Staged = 10;  // after the tiles of gemm_bf16_tiles.hip
+// The kernel a product of contiguous aligned operands runs on (tile, K slices, padded
+// copies); false: a SwiGLU shape without a fused kernel.
+bool plan_gemm_bf16(uint32_t m, uint32_t n, uint32_t k, bool swiglu, bool blocked_a, uint32_t* tile, uint32_t* slices,
+                    bool* padded);
+// One product on a chosen kernel; hipErrorInvalidValue where it cannot run.
+hipError_t launch_gemm_bf16_variant(const uint16_t* a, const uint16_t* b, void* c, uint32_t m, uint32_t n, uint32_t k,
+                                    uint32_t tile, uint32_t slices, bool swiglu, hipStream_t stream);
+// Whether the tile has a SwiGLU form.
+bool bf16_tile_has_swiglu(uint32_t tile);
 // bf16 flash attention, head dim 128, full (non-causal): Q/K/V/O [T, ld*] with
 // head h at column 128 h.  variant 0: K/V tiles moved HBM -> LDS by DMA (64 KiB
 // of dynamic LDS); 1: tiles staged through registers.  hipErrorInvalidValue for

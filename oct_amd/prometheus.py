@@ -60,6 +60,8 @@ DETAIL_INVALID_ARGUMENT = -6906
 DETAIL_SCRATCH_LIMIT = -6930
 DETAIL_SCRATCH_UNAVAILABLE = -6931
 SGEMM_NOALLOC_SCRATCH_BYTES = 64 << 20
+GEMM_BF16_SWIGLU, GEMM_BF16_BLOCKED_A = 1, 2  # flags of the bf16 plan and variant entries
+GEMM_BF16_FIVE_STAGE, GEMM_BF16_STAGED = 9, 10  # kernels after the macro tiles 0-8
 # async and batch (reactor_api.h:84-114, 250-260, 282-295, 1448-1545)
 ASYNC_IDLE, ASYNC_SUBMITTED, ASYNC_READY, ASYNC_FAILED, ASYNC_CONSUMED = range(5)
 DETAIL_ASYNC_NOT_READY = -6108
@@ -897,6 +899,11 @@ _SIGNATURES = {
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, POINTER(c_uint32), POINTER(c_int)]),
     "prometheus_reactor_runtime_gemm_bf16_device": (
         c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, POINTER(c_uint32), POINTER(c_int)]),
+    "prometheus_reactor_gemm_bf16_plan": (
+        c_int, [c_uint32, c_uint32, c_uint32, c_uint32, POINTER(c_uint32), POINTER(c_uint32), POINTER(c_uint32)]),
+    "prometheus_reactor_runtime_gemm_bf16_device_variant": (
+        c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_uint32, c_uint32, c_uint32, c_uint32, c_uint32, c_uint32,
+                POINTER(c_uint32), POINTER(c_int)]),
     "prometheus_reactor_reduction_plan": (
         c_int, [POINTER(PrometheusReductionRequest), POINTER(PrometheusReductionPlan)]),
     "prometheus_reactor_runtime_reduction": (
@@ -1474,6 +1481,15 @@ class NativeRuntime:
                                                                   c_void_p(dc), m, n, k, byref(stage), byref(detail))
         return self._check(rc, stage, detail, "gemm_bf16_device")
 
+    def gemm_bf16_device_variant(self, da: int, db: int, dc: int, m: int, n: int, k: int, tile: int, k_slices: int,
+                                 flags: int = 0) -> Tuple[int, CallStatus]:
+        """One bf16 product on a chosen kernel: (rc, stage/detail); does not raise."""
+        stage, detail = c_uint32(0), c_int(0)
+        rc = self.lib.prometheus_reactor_runtime_gemm_bf16_device_variant(
+            self.handle, c_void_p(da), c_void_p(db), c_void_p(dc), m, n, k, tile, k_slices, flags, byref(stage),
+            byref(detail))
+        return rc, CallStatus(stage.value, detail.value)
+
     def reduction_device(self, din: int, dout: int, rows: int, width: int, operation: int) -> int:
         stage, detail = c_uint32(0), c_int(0)
         rc = self.lib.prometheus_reactor_runtime_reduction_device(self.handle, c_void_p(din), c_void_p(dout), rows,
@@ -1617,6 +1633,15 @@ def sgemm_plan(m: int, n: int, k: int, lib: Optional[ctypes.CDLL] = None) -> Tup
     info.struct_size = ctypes.sizeof(info)
     rc = lib.prometheus_reactor_sgemm_plan(m, n, k, byref(info))
     return rc, info
+
+
+def gemm_bf16_plan(m: int, n: int, k: int, flags: int = 0,
+                   lib: Optional[ctypes.CDLL] = None) -> Optional[Tuple[int, int, bool]]:
+    """The kernel of a bf16 product (no device needed): (tile, K slices, padded copies), or None."""
+    lib = lib or shared_library()
+    tile, slices, padded = c_uint32(0), c_uint32(0), c_uint32(0)
+    rc = lib.prometheus_reactor_gemm_bf16_plan(m, n, k, flags, byref(tile), byref(slices), byref(padded))
+    return (tile.value, slices.value, padded.value != 0) if rc == PROM_OK else None
 
 
 # ---- the strict `@` path (strict.go:11-32, runtime.go:251-317) -------------

@@ -314,9 +314,9 @@ def test_bf16_4096_cubed(gpu_runtime):
 @pytest.mark.parametrize("m,n,k", [(4224, 2056, 72), (600, 8200, 136), (1024, 4096, 8),
                                    (1100, 16400, 96), (2560, 3584, 8224)])
 def test_bf16_large_tile_kernel_ragged(gpu_runtime, m, n, k):
-    """Shapes with >= 128 256x256 tiles take the large-tile kernels; ragged m/n/k tails.
-    (1100, 16400, 96) and (2560, 3584, 8224) take the four-stage kernel (more
-    than 256 tiles, or K >= 8192; K a multiple of 32 but not of 64)."""
+    """Ragged m/n/k tails on the larger macro tiles the plan picks here: 192x256, 128x256,
+    64x128, 192x256 and 192x128 (test_gemm_bf16_plan.py; the five-stage 256x256 kernel's
+    ragged shapes are in test_gpu_gemm_bf16_tiles.py)."""
     a = oracle.to_bf16(oracle.uniform(50 + m, (m, k)))
     b = oracle.to_bf16(oracle.uniform(60 + n, (k, n)))
     out = gpu_runtime.gemm_bf16(m, n, k, a, b).reshape(m, n)
