@@ -179,7 +179,7 @@ struct SgemmRowsPlan {
   int shape, splits;
   double us;
 };
-bool sgemm_rows_take(uint32_t m, uint32_t k, int lda, int ldb, int halves);
+bool sgemm_rows_take(uint32_t m, uint32_t k, int lda, int ldb);
 SgemmRowsPlan plan_sgemm_rows(uint32_t m, uint32_t n, uint32_t k, bool geglu, uint64_t max_partial_floats);
 int sgemm_rows_columns(const SgemmRowsPlan& plan);
 hipError_t launch_sgemm_rows(const SgemmRowsPlan& plan, const float* a, int lda, const float* b, int ldb, float* c,

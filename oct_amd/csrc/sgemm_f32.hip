@@ -1347,7 +1347,7 @@ uint64_t sliced_floats(int splits, uint32_t m, uint32_t n) { return splits > 1 ?
 // outgrow the allocation-free scratch (45x67176x7772: 6, 69 MiB) give way to fewer.
 bool few_rows_win(uint32_t m, uint32_t n, uint32_t k, int lda, int ldb, double tiles_us, uint64_t max_partial_floats,
                   SgemmRowsPlan* rows) {
-  if (!sgemm_rows_take(m, k, lda, ldb, 1)) return false;
+  if (!sgemm_rows_take(m, k, lda, ldb)) return false;
   *rows = plan_sgemm_rows(m, n, k, false, max_partial_floats);
   if (sliced_floats(rows->splits, m, n) > kNoallocFloats) {
     const SgemmRowsPlan fits = plan_sgemm_rows(m, n, k, false, std::min(max_partial_floats, kNoallocFloats));
@@ -1677,16 +1677,19 @@ hipError_t launch_sgemm_f32_geglu(const float* a, int lda, const float* w, float
                                   uint32_t k, hipStream_t stream) {
   if (m == 0 || f == 0 || k == 0) return hipErrorNotSupported;
   const int ldb = (int)(2 * f);
+  const bool tiles = f % 64 == 0 && k % kBK == 0 && ldh % 4 == 0 && aligned16(h) &&
+                     buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k);
   // Few rows: the tiles would run most of theirs as padding (15 rows of the Gemma
-  // layer's 2048 x 2 * 16384: 132 us).
-  if (sgemm_rows_take(m, k, lda, ldb, 2)) {
+  // layer's 2048 x 2 * 16384: 132 us), but win back the few-rows kernel's reading rate
+  // for 33 rows and more of a very wide product (a layer of 48 tokens, F = 81920: 555 us
+  // with few rows, 539 with tiles; F = 16384: 159 and 175).  The 64-row tile, which
+  // geglu_height takes for them, is priced as the plain product's.
+  if (sgemm_rows_take(m, k, lda, ldb)) {
     const SgemmRowsPlan rows = plan_sgemm_rows(m, f, k, true, 0);
-    const double tiles = plan_cost(SgemmPlan{4, 1, (int)k}, m, 2 * f, 1);
-    if (rows.us < tiles) return launch_sgemm_rows_geglu(rows, a, lda, w, h, ldh, m, f, k, stream);
+    if (!tiles || rows.us < plan_cost(SgemmPlan{7, 1, (int)k}, m, 2 * f, 1))
+      return launch_sgemm_rows_geglu(rows, a, lda, w, h, ldh, m, f, k, stream);
   }
-  const bool ok = f % 64 == 0 && k % kBK == 0 && ldh % 4 == 0 && aligned16(h) &&
-                  buffer_path(aligned16(a) && aligned16(w), lda, 0, ldb, 0, m, 2 * f, k);
-  if (!ok) return hipErrorNotSupported;
+  if (!tiles) return hipErrorNotSupported;
   switch (geglu_height(m)) {
     case 64: launch_geglu_tiles<64>(a, lda, w, h, ldh, m, f, k, stream); break;
     case 192: launch_geglu_tiles<192>(a, lda, w, h, ldh, m, f, k, stream); break;

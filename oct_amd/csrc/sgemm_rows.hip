@@ -260,9 +260,9 @@ hipError_t launch_rows_of(int shape, int splits, const RowsArgs& p, hipStream_t 
 
 }  // namespace
 
-bool sgemm_rows_take(uint32_t m, uint32_t k, int lda, int ldb, int halves) {
+bool sgemm_rows_take(uint32_t m, uint32_t k, int lda, int ldb) {
   const size_t lim = (1ull << 31) - (1u << 16);
-  return m <= 48u && (size_t)m * lda * 4 < lim && ((size_t)k + 32) * ldb * 4 < lim && halves >= 1;
+  return m <= 48u && (size_t)m * lda * 4 < lim && ((size_t)k + 32) * ldb * 4 < lim;
 }
 
 SgemmRowsPlan plan_sgemm_rows(uint32_t m, uint32_t n, uint32_t k, bool geglu, uint64_t max_partial_floats) {
