@@ -646,7 +646,10 @@ int swiglu_tail_splits(uint32_t m, uint32_t f, uint32_t k) {
 
 // True when the SwiGLU GEMM runs on the five-stage kernel, as bf16_path decides.  Where
 // its final wave is split along K the estimate, which adds the waves up, is too
-// high (dispatch overlaps them), so there the tiles have to be 30 % better.
+// high (dispatch overlaps them), so there the tiles have to be 30 % better.  That holds
+// for 3840 wide blocks (2320 tokens 967 us, on tiles 986; 2384: 977 and 993), which the
+// figure is drawn for; narrower ones would gain from the tiles (2048 wide, 1296 tokens: 286 us,
+// on tiles 261; 3072 wide, 528: 280 and 260; 1024 wide, 3024: 229 and 209).
 bool swiglu_five_stage(const uint16_t* a, int lda, const uint16_t* w13, uint32_t m, uint32_t f, uint32_t k) {
   if (!swiglu_five_stage_ok(a, lda, w13, m, f, k)) return false;
   const int splits = swiglu_tail_splits(m, f, k);

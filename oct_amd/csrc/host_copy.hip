@@ -13,7 +13,8 @@
 //     copying (3 copies of 64 KiB and a kernel: 38 us by DMA, 22 by kernels);
 //   * larger ones in chunks of half the copy, 1 to 8 MiB: the host threads copy
 //     chunk i into a pinned slot while chunk i-1 moves, and the reverse for
-//     downloads.  Four host threads (the caller and three workers) copy pageable
+//     downloads (a slot is written again only when an event behind every copy from it
+//     has passed: Ring).  Four host threads (the caller and three workers) copy pageable
 //     <-> pinned at 70-95 GB/s (one: 30); the pipelined upload of 64 MiB measured 47
 //     GB/s.  Two chunks keep a copy of a few MiB, which was one, from running host
 //     and device in turn; below 4 MiB they move by the copy kernel too, since each

@@ -1341,9 +1341,13 @@ constexpr double kFitsWithin = 1.02;
 uint64_t sliced_floats(int splits, uint32_t m, uint32_t n) { return splits > 1 ? (uint64_t)splits * m * n : 0; }
 
 // Whether the few-rows kernel takes an m x n x k product that the tiles are estimated
-// to run in tiles_us.  The two models meet where both are off: a sliced product of a
-// small B measured slower than the tiles (24x256x1536: 9.9 us against 8.9), a larger
-// one faster (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).  Slices that
+// to run in tiles_us.  The two models meet where both are off, so near a tie a sliced
+// product of a small B has 1.6 us added (24x256x1536 measured 9.9 us against 8.9) and a
+// larger one 6 % taken off (33x2048x2048, both estimated 11.8: rows 10.0, tiles 12.4).
+// At 160 random products of 1 to 48 rows (n 64..16384, k 64..8192) this took the few-rows
+// kernel every time: 1.48 times faster in the median, 1 % slower at worst, with B in the
+// caches; from HBM 1.52 times, and slower at two (11x2816x7360 40.0 us against 32.5,
+// 27x1152x1472 10.6 against 9.5).  Slices that
 // outgrow the allocation-free scratch (45x67176x7772: 6, 69 MiB) give way to fewer.
 bool few_rows_win(uint32_t m, uint32_t n, uint32_t k, int lda, int ldb, double tiles_us, uint64_t max_partial_floats,
                   SgemmRowsPlan* rows) {
@@ -1400,7 +1404,10 @@ SgemmSchedule schedule_products(bool aligned, int lda, int ldb, uint32_t m, uint
       q.tail = plan_rows(tail_aligned, tail, max_floats);
       double tail_us = plan_cost(q.tail, tail, n, 1, kind);
       // The few-rows kernel takes short K's tails, which the tiles cannot slice (one row
-      // of 3001x516: 5.5 us against 10); a long K's are 1 or 2 % of the whole either way.
+      // of 3001x516: 5.5 us against 10).  A longer K's stay on the tiles, where the limit
+      // was drawn with little to choose; 40 products of k 1040..7984 with such a tail
+      // measured 3.4 % faster in the median with it on the few-rows kernel
+      // (2059x512x1040: 31.2 -> 26.1 us), one 2.4 % slower.
       q.tail_rows = k < 1024u && few_rows_win(tail, n, k, lda, ldb, tail_us, max_floats, &q.rows);
       if (q.tail_rows) tail_us = q.rows.us;
       q.us = plan_cost(q.head, head, n, 1, kind) + tail_us;

@@ -53,8 +53,12 @@ struct RowsShape {
 // granule (0.72 of it more per further 16 rows, the matrix cores' share), each wave
 // through its own at `chain`, and B arrives at 6.2 TB/s at most.  The plan with the
 // least estimate is within 4 % of the fastest measured on average, 27 % at worst
-// (1x1418x4315).  us, the tiles of sgemm_f32.hip -> this: 15x2048x1536 9.9 -> 7.7,
-// 15x8192x2048 22.3 -> 12.7, 15x32768x2048 67.7 -> 47.5, 48x16384x8192 156 -> 127.
+// (1x1418x4315); those runs' operands were in the caches.  us, the tiles of
+// sgemm_f32.hip -> this, with B in the caches and, in brackets, with 1.2 GB of matrices in
+// turn: 15x2048x1536 9.4 -> 5.5 (10.7 -> 10.5), 15x8192x2048 22.2 -> 11.9 (23.4 -> 15.0),
+// 15x32768x2048 64.2 -> 40.9 (67.3 -> 49.7), 48x16384x8192 148 -> 118 (148 -> 118).
+// Against a B that comes from HBM the estimate is low: by 9 % in the median of 160
+// products, 26 % at the ninth decile.
 constexpr RowsShape kShapes[] = {{1, 8, 0.0344, 0.305}, {1, 16, 0.0345, 0.491}, {2, 8, 0.0485, 0.385},
                                  {2, 16, 0.0512, 0.333}, {4, 4, 0.0916, 0.555}, {4, 8, 0.0897, 0.566}};
 constexpr int kNumShapes = sizeof(kShapes) / sizeof(kShapes[0]);
@@ -169,8 +173,8 @@ __global__ __launch_bounds__(64 * kW) void sgemm_rows_kernel(const RowsArgs p) {
   };
 
   // The wave's granules are g0 + wave, then every kW-th; the next one's loads are in
-  // flight while one is multiplied (two ahead measured no faster: the other waves of
-  // the CU cover the rest).
+  // flight while one is multiplied (two ahead measured 0 to 5 % slower at nine products,
+  // with B in the caches and from HBM alike: the other waves of the CU cover the rest).
   Granule q;
   int g = g0 + wave;
   if (g < g1) load(q, g);
