@@ -62,6 +62,20 @@ def test_staged_tiles_at_any_alignment(gpu_runtime, tile, slices, m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 6, 7, 103, 1025, 1027])
+def test_sums_of_slices_for_any_column_count(gpu_runtime, n):
+    """The slices' sum takes four columns per thread, the last ones together with columns that
+    another thread stores, and one per thread below four; 130 rows of 13 slices."""
+    rt = gpu_runtime
+    m, k = 130, 1040
+
+    def run(a, b, c):
+        assert rt.sgemm_device_variant(a, b, c, m, n, k, 2, 13)[0] == p.PROM_OK
+
+    _check(rt, m, n, k, run)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("m,n,k", [(256, 256, 20), (640, 640, 1032), (384, 2304, 124), (129, 128, 516),
                                    (2944, 2816, 60)])
 def test_k_tail_of_aligned_operands(gpu_runtime, m, n, k):
